@@ -1330,25 +1330,45 @@ __global__ __launch_bounds__(256) void k_update(DevPtrs<R> p, double Rgas, doubl
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const int c = tile * 256 + threadIdx.x;
     if (c >= p.nc) return;
-    const int C = p.ccnt[c], maxC = p.maxC, nf = p.nf;
-    const double dt = dt_ptr ? dt_ptr[p.cinst ? p.cinst[c] : 0] : dt_val;
-    if (dt_ptr && dt == 0.0) return;  // device path past its end time: the state stays
-    double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
-    for (int fi = 0; fi < C; ++fi) {
-        const int sf = p.slot_face[sell(c, fi, maxC)];
-        const int dir = (sf > 0) - (sf < 0);
-        const int f = (sf < 0 ? -sf : sf) - 1;
-        const double4 F = face_flux(p, f);
-        r0 += dir * F.x;
-        r1 += dir * F.y;
-        r2 += dir * F.z;
-        r3 += dir * F.w;
-    }
+    const int maxC = p.maxC, nf = p.nf;
+    // Bound by its loads.  The first PF slots' faces are requested at once, then
+    // their fluxes, so that a cell waits for two memory rounds and not for two
+    // per face; a padding slot (0) reads face 0 and is left out of the sums.
+    // Back to back on 1.5M cells 55.7 -> 48.1 us (FP64), 250k quads 12.9 ->
+    // 10.8, 20k quads 5.2 -> 4.7 (a launch that only reduces 157 values takes 2.5).
+    constexpr int PF = 4;
+    int sfs[PF];
+#pragma unroll
+    for (int fi = 0; fi < PF; ++fi) sfs[fi] = fi < maxC ? p.slot_face[sell(c, fi, maxC)] : 0;
+    const int C = p.ccnt[c];
     const double V = p.vol[c];
     // b2 = 0 (first stage): U equals Uold at the start of every step (both
     // are stored from one value at the end of a step and at upload), so the
     // stage reads it once; b2 * u is then b2 * uo, the same value
     const double4 uo = p.Uold[c], u = b2 == 0.0 ? uo : p.U[c];
+    const double dt = dt_ptr ? dt_ptr[p.cinst ? p.cinst[c] : 0] : dt_val;
+    double4 F[PF];
+#pragma unroll
+    for (int fi = 0; fi < PF; ++fi) {
+        const int f = max((sfs[fi] < 0 ? -sfs[fi] : sfs[fi]) - 1, 0);
+        F[fi] = face_flux(p, f);
+    }
+    if (dt_ptr && dt == 0.0) return;  // device path past its end time: the state stays
+    double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
+    auto add = [&](int sf, const double4& Fs) {
+        const int dir = (sf > 0) - (sf < 0);
+        r0 += dir * Fs.x;
+        r1 += dir * Fs.y;
+        r2 += dir * Fs.z;
+        r3 += dir * Fs.w;
+    };
+#pragma unroll
+    for (int fi = 0; fi < PF; ++fi)
+        if (sfs[fi] != 0) add(sfs[fi], F[fi]);
+    for (int fi = PF; fi < C; ++fi) {
+        const int sf = p.slot_face[sell(c, fi, maxC)];
+        add(sf, face_flux(p, (sf < 0 ? -sf : sf) - 1));
+    }
     const double rho = b1 * uo.x + b2 * u.x + b3 * dt * (-r0 / V);
     const double rhoUx = b1 * uo.y + b2 * u.y + b3 * dt * (-r1 / V);
     const double rhoUy = b1 * uo.z + b2 * u.z + b3 * dt * (-r2 / V);
@@ -1371,10 +1391,9 @@ __global__ __launch_bounds__(256) void k_update(DevPtrs<R> p, double Rgas, doubl
     wr.w = (R)w.w;
     p.W[c] = wr;
     // ghost states of this cell's boundary faces (K10), from the updated state
-    for (int fi = 0; fi < C; ++fi) {
-        const int sf = p.slot_face[sell(c, fi, maxC)];
+    auto ghost = [&](int sf) {
         const int f = sf - 1;
-        if (f < nf) continue;
+        if (f < nf) return;
         const int b = f - nf;
         const double4 g = boundary_value(p.blabel[b], w, p.bgeo[b], p.bval[b]);
         typename VT<R>::v4 gr;
@@ -1383,7 +1402,10 @@ __global__ __launch_bounds__(256) void k_update(DevPtrs<R> p, double Rgas, doubl
         gr.z = (R)g.z;
         gr.w = (R)g.w;
         p.W[p.nc + b] = gr;
-    }
+    };
+#pragma unroll
+    for (int fi = 0; fi < PF; ++fi) ghost(sfs[fi]);
+    for (int fi = PF; fi < C; ++fi) ghost(p.slot_face[sell(c, fi, maxC)]);
 }
 
 // ---------------------------------------------------------------- launchers
