@@ -77,6 +77,11 @@ def render(c):
         lines.append("    b0_ = (tt_ * b1_ - b2_) + %sf; b2_ = b1_; b1_ = b0_; \\" % repr(float(c[k])))
     lines.append("    (out) = ((t) * b1_ - b2_) + %sf; \\" % repr(float(c[0])))
     lines.append("} while (0)")
+    lines.append("// The coefficients of both series, from the highest degree down.")
+    for name, top, suffix in (("AFAR_ERFCX", n, ""), ("AFAR_ERFCX_F", m, "f")):
+        lines += ["#define %s_COUNT %d" % (name, top + 1), "#define %s_COEFFS { \\" % name]
+        lines += ["    %s%s, \\" % (repr(float(c[k])), suffix) for k in range(top, -1, -1)]
+        lines.append("}")
     return "\n".join(lines) + "\n"
 
 
