@@ -40,7 +40,8 @@ struct DevPtrs {
     uint8_t* flat_prev;        // nc: the cell took the flat branch at the last reconstruction (load scheduling only)
     const uint8_t* scnt;       // nc stencil size
     const uint8_t* ccnt;       // nc compact stencil size
-    const uint16_t* sten;      // sliced ELL, LDS-local stencil ids
+    int stenW;                 // ids per row of sten, a multiple of 8
+    const uint16_t* sten;      // one row per cell: LDS-local stencil ids, then the dummy member's
     const int32_t* slot_face;  // sliced ELL, +-(face+1)
     const typename VT<R>::v2* slot_d;  // sliced ELL, face centre - cell centre, in the kernels' precision
     const double2* slot_e;     // sliced ELL, compact neighbour - cell centre (K3 only)
@@ -58,8 +59,10 @@ struct DevPtrs {
     R* slot_dr;                // sliced ELL, |slot_e| in the kernels' precision (written by K3)
     typename VT<R>::v2* lsq;   // sliced ELL, least-squares weights
     const R* rbf;              // sliced ELL, RBF coefficients (face slot, stencil member)
-    const int32_t* halo_ptr;
-    const int32_t* halo;
+    int hfix, hcap;            // halo ids per row, capacity of the LDS halo (the dummy member follows it)
+    const int32_t* halo;       // ntiles rows of hfix ids
+    const int32_t* more_ptr;   // ntiles+1, ids of the longer lists past their row
+    const int32_t* halo_more;
     const int2* fcell;         // nf own, nei
     const double4* fgeo;       // 2*nf: (Sfx, Sfy, magSf, deltaR), (dxo, dyo, dxn, dyn)
     const float4* fgeo32;      // FP32-mixed: fgeo rounded to float (the flux pass without the CFL bound

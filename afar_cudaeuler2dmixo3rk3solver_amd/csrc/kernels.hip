@@ -159,18 +159,18 @@ __global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double R_, double Cv,
 
 // ---------------------------------------------------------------- K5 reconstruct
 
-// Copies the stencil ids (sliced ELL, width 64) of the tile's cells into LDS:
-// the tile's waves are consecutive slices, so the block is one contiguous
-// range of (waves of the tile) * maxS * 64 ids, copied 16 bytes at a time.
-__device__ __forceinline__ void stage_stencil(uint16_t* sSt, const uint16_t* sten, int tile, int tileCells, int nc,
-                                              int maxS, int t, int nthreads) {
+// 16-byte words of the tile's block of stencil ids (one row of stenW ids per cell).
+__device__ __forceinline__ int sten_words(int tile, int tileCells, int nc, int stenW) {
     const int wpt = tileCells >> 6;  // waves per tile
-    const int w0 = tile * wpt;
-    const int nw = min(wpt, ((nc + 63) >> 6) - w0);
-    const int n16 = nw * maxS * 8;  // 16-byte words (64 ids of 2 bytes = 8 words per slice row)
-    const uint4* src = reinterpret_cast<const uint4*>(sten + (size_t)w0 * maxS * 64);
-    uint4* dst = reinterpret_cast<uint4*>(sSt);
-    for (int i = t; i < n16; i += nthreads) dst[i] = src[i];
+    return min(wpt, ((nc + 63) >> 6) - tile * wpt) * 8 * stenW;
+}
+
+// The tile's halo members into LDS slots TILE..: fn(slot, id).
+template <int TILE, typename R, typename F>
+__device__ __forceinline__ void stage_halo(const DevPtrs<R>& p, int tile, int t, int nthreads, F fn) {
+    for (int i = t; i < p.hfix; i += nthreads) fn(TILE + i, p.halo[(size_t)tile * p.hfix + i]);
+    const int m0 = p.more_ptr[tile], m1 = p.more_ptr[tile + 1];
+    for (int i = m0 + t; i < m1; i += nthreads) fn(TILE + p.hfix + i - m0, p.halo_more[i]);
 }
 
 // The reconstructed state of face side i (= 2f + side): FP64 one array per
@@ -216,13 +216,17 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     if (tile >= p.ntiles) return;
     const int tid = threadIdx.x, c = tile * TILE + tid;
-    const int hb = p.halo_ptr[tile], hn = p.halo_ptr[tile + 1] - hb;
-    uint16_t* sSt = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
+    uint16_t* sRows = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
     if (c < p.nc) sW[tid] = p.W[c];
-    for (int i = tid; i < hn; i += TILE) sW[TILE + i] = p.W[p.halo[hb + i]];
-    stage_stencil(sSt, p.sten, tile, TILE, p.nc, p.maxS, tid, TILE);
+    stage_halo<TILE>(p, tile, tid, TILE, [&](int j, int id) { sW[j] = p.W[id]; });
+    {
+        const uint4* src = reinterpret_cast<const uint4*>(p.sten + (size_t)tile * TILE * p.stenW);
+        const int n16 = sten_words(tile, TILE, p.nc, p.stenW);
+        for (int i = tid; i < n16; i += TILE) reinterpret_cast<uint4*>(sRows)[i] = src[i];
+    }
     __syncthreads();
     if (c >= p.nc) return;
+    const uint16_t* sSt = sRows + tid * p.stenW;  // this cell's members
     const int S = p.scnt[c], C = p.ccnt[c];
     const int maxS = p.maxS, maxC = p.maxC, KR = maxC * (maxS + 1);
     const v4 wc = sW[tid];
@@ -230,7 +234,7 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
     R gpx = 0, gpy = 0, guxx = 0, guyx = 0, guxy = 0, guyy = 0, gTx = 0, gTy = 0;
     for (int i = 0; i < C; ++i) {
         const v2 M = p.lsq[sell(c, i, maxC)];
-        const v4 wj = sW[sSt[sell(tid, i, maxS)]];
+        const v4 wj = sW[sSt[i]];
         R dphi = wj.x - wc.x;
         gpx += M.x * dphi;
         gpy += M.y * dphi;
@@ -251,7 +255,7 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
 
     R pMax = wc.x, pMin = wc.x, uxMax = wc.y, uxMin = wc.y, uyMax = wc.z, uyMin = wc.z, TMax = wc.w, TMin = wc.w;
     for (int i = 0; i < C; ++i) {
-        const v4 wj = sW[sSt[sell(tid, i, maxS)]];
+        const v4 wj = sW[sSt[i]];
         pMax = fmax(wj.x, pMax);
         pMin = fmin(wj.x, pMin);
         uxMax = fmax(wj.y, uxMax);
@@ -310,13 +314,13 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
         const R dx = d.x, dy = d.y;
         const R deltaR = p.slot_dr[sell(c, fi, maxC)];
         const R fraction = sqrt(dx * dx + dy * dy) / deltaR;
-        const int nbl = sSt[sell(tid, fi, maxS)];
+        const int nbl = sSt[fi];
 
         const R* a = p.rbf + sell(c, fi * (maxS + 1), KR);  // row stride 64
         R coef = a[0];
         R pf = coef * wc.x, uxf = coef * wc.y, uyf = coef * wc.z, Tf = coef * wc.w;
         for (int ci = 0; ci < S; ++ci) {
-            const v4 wj = sW[sSt[sell(tid, ci, maxS)]];
+            const v4 wj = sW[sSt[ci]];
             coef = a[(size_t)(ci + 1) * 64];
             pf += coef * wj.x;
             uxf += coef * wj.y;
@@ -344,7 +348,7 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
             R cg = ag[0];
             R pg = cg * wc.x, uxg = cg * wc.y, uyg = cg * wc.z, Tg = cg * wc.w;
             for (int ci = 0; ci < S; ++ci) {
-                const v4 wj = sW[sSt[sell(tid, ci, maxS)]];
+                const v4 wj = sW[sSt[ci]];
                 cg = ag[(size_t)(ci + 1) * 64];
                 pg += cg * wj.x;
                 uxg += cg * wj.y;
@@ -400,6 +404,16 @@ template <int X, typename T> __device__ __forceinline__ T quad_xor(T x) {
     return dpp_move<X == 1 ? 0xB1 : 0x4E>(x);  // quad_perm [1,0,3,2] and [2,3,0,1]
 }
 
+// The largest of the values below 32 that x has in the lanes where m holds (0
+// if there is none): the same in every lane.
+__device__ __forceinline__ int wave_max32(int x, bool m) {
+    int r = 0;
+#pragma unroll
+    for (int b = 16; b > 0; b >>= 1)
+        if (__ballot(m && x >= r + b) != 0) r += b;
+    return r;
+}
+
 // K5 with four lanes per cell, for meshes whose cells have at most four
 // faces (triangles and quads): lane k of a cell's group handles face slot k
 // (its RBF sum and limiter candidates) and variable k of the gradient and the
@@ -407,24 +421,36 @@ template <int X, typename T> __device__ __forceinline__ T quad_xor(T x) {
 // exact reductions over the group (the limiter is a minimum, the smoothness a
 // maximum, the trouble test that of the last internal face), so the values
 // equal the one-lane-per-cell kernel's bit for bit.
-// Waves per SIMD the register allocator must allow for the four-lane kernel,
-// per working type (build-time tuning knobs; 1 = no constraint).  5 (FP64, 96
-// VGPRs) and 8 (FP32, 64 VGPRs) fit without spills and were measured faster
-// than the unconstrained 4 and 7 waves.
+// MS bounds the stencil size (8: quads, 16: mixed triangles and quads, 20), so
+// that meshes of short stencils hold fewer coefficients in registers.
+//
+// Bound by its chain of loads and LDS reads on small meshes (15.8k cycles per
+// wave before the following), by the memory it writes and by VALU issue on
+// large ones.  No step of the chain waits alone: halo ids lie in rows of fixed
+// width (no offset to wait for), slots are read without their count, a cell's
+// member ids are one or two 16-byte words, and the RBF sums run to the
+// wavefront's longest stencil with terms that add nothing past a cell's own.
+// Back to back: 800 cells 8.3 -> 6.2 us, 20k quads 10.1 -> 8.4 (mixed 7.9 ->
+// 6.5), 17k periodic quads 9.7 -> 8.3, 524k mixed 44.1 -> 41.1; 1.5M triangles
+// and quads 221 -> 220.
+// Waves per SIMD the register allocator must allow, per working type
+// (build-time tuning knobs; 1 = no constraint).  At 5 (FP64) and 8 (FP32) the
+// 16-member kernels spill 5 values and 1: Riemann 233 us instead of 220, and
+// 84.4 instead of 81.2 (mixed, 740k cells).
 #ifndef AFAR_RECONQ_WPE_D
-#define AFAR_RECONQ_WPE_D 5
+#define AFAR_RECONQ_WPE_D 4
 #endif
 #ifndef AFAR_RECONQ_WPE_F
-#define AFAR_RECONQ_WPE_F 8
+#define AFAR_RECONQ_WPE_F 7
 #endif
-// The flux-quadrature instantiation holds more values and asks for one wave
-// fewer, so that it does not spill.
+// The float flux-quadrature instantiation holds more values and asks for one
+// wave fewer, so that it does not spill.
 template <typename R, bool GP> struct ReconQWaves {
-    static constexpr int value = (sizeof(R) == 8 ? AFAR_RECONQ_WPE_D : AFAR_RECONQ_WPE_F) - (GP ? 1 : 0);
+    static constexpr int value = sizeof(R) == 8 ? AFAR_RECONQ_WPE_D : AFAR_RECONQ_WPE_F - (GP ? 1 : 0);
 };
 #define AFAR_RECONQ_ATTR __attribute__((amdgpu_waves_per_eu(ReconQWaves<R, GP>::value, 8)))
 
-template <typename R, int TILE, bool GP>
+template <typename R, int TILE, bool GP, int MS>
 __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(DevPtrs<R> p) {
     using v4 = typename VT<R>::v4;
     using v2 = typename VT<R>::v2;
@@ -437,169 +463,184 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     constexpr bool GEO = sizeof(R) == 8 && !GP;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     v4* sW = reinterpret_cast<v4*>(smem_raw);
+    uint16_t* sRows = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
+    v2* sM = reinterpret_cast<v2*>(smem_raw + p.lds_m_off);            // 4 weights per cell
+    double2* sC = reinterpret_cast<double2*>(smem_raw + p.lds_m_off);  // GEO: tile + halo centres instead
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     if (tile >= p.ntiles) return;
     const int t = threadIdx.x;
     const int lc = t >> 2, k = t & 3;
     const int c = tile * TILE + lc;
-    const int maxS = p.maxS, maxC = p.maxC, KR = maxC * (maxS + 1), nf = p.nf;
+    const int maxC = p.maxC, KR = maxC * (p.maxS + 1), nf = p.nf, SW = p.stenW;
     // Every load that needs no LDS is issued before the staging barrier, in
-    // two dependent rounds: (1) the cell's counts, the tile's own states,
-    // halo ids and stencil block; (2) lane k's least-squares weight and slot
-    // data, and the halo states.  Their latencies overlap.
+    // two dependent rounds: (1) the cell's counts, lane k's slot, the tile's
+    // own states, halo ids and stencil rows; (2) the halo states, the slot's
+    // face centre and, where the full path is foreseen, its RBF coefficients.
     const bool inb = c < p.nc;
     int S = 0, C = 0, sf = 0, wasFlat = 0;
     if (inb) {
         S = p.scnt[c];
         C = p.ccnt[c];
         wasFlat = p.flat_prev[c];
+        if (k < maxC) sf = p.slot_face[sell(c, k, maxC)];  // 0: no such slot
     }
-    const int hb = p.halo_ptr[tile], hn = p.halo_ptr[tile + 1] - hb;
-    const int wpt = TILE >> 6;  // stencil block: (waves of the tile) * maxS * 64 ids
-    const int nw = min(wpt, ((p.nc + 63) >> 6) - tile * wpt);
-    const int n16 = nw * maxS * 8;
-    const uint4* stSrc = reinterpret_cast<const uint4*>(p.sten + (size_t)tile * wpt * maxS * 64);
+    const int n16 = sten_words(tile, TILE, p.nc, SW);
+    const uint4* stSrc = reinterpret_cast<const uint4*>(p.sten + (size_t)tile * TILE * SW);
     const bool ownW = t < TILE && tile * TILE + t < p.nc;
-    v4 wOwn;
-    if (ownW) wOwn = p.W[tile * TILE + t];
+    const bool ownH = t < p.hfix;
+    v4 wOwn, wHalo;
+    double2 cOwn, cHalo;  // GEO: staged centres
     uint4 st0;
-    if (t < n16) st0 = stSrc[t];
     int h0 = 0;
-    if (t < hn) h0 = p.halo[hb + t];
+    if (ownH) h0 = p.halo[(size_t)tile * p.hfix + t];
+    if (ownW) {
+        wOwn = p.W[tile * TILE + t];
+        if constexpr (GEO) cOwn = p.cen[tile * TILE + t];
+    }
+    if (t < n16) st0 = stSrc[t];
+    const int m0 = p.more_ptr[tile], m1 = p.more_ptr[tile + 1];
+    if (ownH) {
+        wHalo = p.W[h0];
+        if constexpr (GEO) cHalo = p.cen[h0];
+    }
+    const int isNei = sf < 0;
+    const int f = (sf < 0 ? -sf : sf) - 1;
+    const bool has = sf != 0, live = has && f < nf;
     v2 Mk = v2{(R)0, (R)0};
     v2 d = v2{(R)0, (R)0};
-    if (inb && k < C) {
-        sf = p.slot_face[sell(c, k, maxC)];
-        if constexpr (!GEO) {
+    double2 fc = double2{0.0, 0.0}, fs = double2{0.0, 0.0};  // GEO: face centre, periodic shift
+    if (has) {
+        if constexpr (GEO) {
+            fc = p.fcen[f];
+            if (p.fshift && live) fs = p.fshift[f];
+        } else {
             Mk = p.lsq[sell(c, k, maxC)];
             d = p.slot_d[sell(c, k, maxC)];
         }
     }
-    v4 wHalo;
-    if (t < hn) wHalo = p.W[h0];
-    double2 cOwn = double2{0.0, 0.0}, cHalo = double2{0.0, 0.0};  // GEO: staged centres
-    double2 fc = double2{0.0, 0.0}, fs = double2{0.0, 0.0};        // GEO: face centre, periodic shift
-    if constexpr (GEO) {
-        if (ownW) cOwn = p.cen[tile * TILE + t];
-        if (t < hn) cHalo = p.cen[h0];
-        if (inb && k < C) {
-            const int ff = (sf < 0 ? -sf : sf) - 1;
-            fc = p.fcen[ff];
-            if (p.fshift && ff < nf) fs = p.fshift[ff];
-        }
-    }
     // A cell that took the full path at the previous launch most likely takes
     // it again: its RBF coefficients and centre distance are requested in this
-    // round already (flat_prev only schedules loads; results do not depend on it).
-    R cf[kMaxSten + 1];
+    // round already (flat_prev only schedules loads; results do not depend on
+    // it).  The row count is the wavefront's: a cell of a shorter stencil reads
+    // its padding (-0.0), which shares the other cells' 128-byte segments.
+    R cf[MS + 1];
     R deltaR = 0;
-    const R* a = p.rbf + sell(c, k * (maxS + 1), KR);  // row stride 64
-    const bool early = inb && k < C && !wasFlat;
-    if (early) {
-        if constexpr (!GEO) deltaR = p.slot_dr[sell(c, k, maxC)];
+    const R* a = p.rbf + sell(c, k * (p.maxS + 1), KR);  // row stride 64
 #pragma unroll
-        for (int i = 0; i <= kMaxSten; ++i)
-            if (i <= S) cf[i] = a[(size_t)i * 64];
+    for (int i = 0; i <= MS; ++i) cf[i] = (R)-0.0;
+    auto load_coefficients = [&](bool need) {
+        const int rows = wave_max32(S, need);
+        if (need) {
+            if constexpr (!GEO) deltaR = p.slot_dr[sell(c, k, maxC)];
+#pragma unroll
+            for (int i = 0; i <= MS; ++i)
+                if (i <= rows) cf[i] = a[(size_t)i * 64];
+        }
+    };
+    const bool early = live && !wasFlat;
+    load_coefficients(early);
+    uint4* stDst = reinterpret_cast<uint4*>(sRows);
+    if (ownW) {
+        sW[t] = wOwn;
+        if constexpr (GEO) sC[t] = cOwn;
     }
-    uint16_t* sSt = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
-    v2* sM = reinterpret_cast<v2*>(smem_raw + p.lds_m_off);  // 4 weights per cell
-    double2* sC = reinterpret_cast<double2*>(smem_raw + p.lds_m_off);  // GEO: tile + halo centres instead
-    uint4* stDst = reinterpret_cast<uint4*>(sSt);
-    if (ownW) sW[t] = wOwn;
-    if (t < hn) sW[TILE + t] = wHalo;
+    if (ownH) {
+        sW[TILE + t] = wHalo;
+        if constexpr (GEO) sC[TILE + t] = cHalo;
+    }
     if (t < n16) stDst[t] = st0;
-    if constexpr (GEO) {
-        if (ownW) sC[t] = cOwn;
-        if (t < hn) sC[TILE + t] = cHalo;
-        for (int i = t + NT; i < hn; i += NT) sC[TILE + i] = p.cen[p.halo[hb + i]];
-    } else {
-        sM[t] = Mk;
-    }
-    for (int i = t + NT; i < hn; i += NT) sW[TILE + i] = p.W[p.halo[hb + i]];  // halos beyond NT cells
+    if constexpr (!GEO) sM[t] = Mk;
+    if (t == NT - 1) sW[TILE + p.hcap] = v4{(R)1, (R)1, (R)1, (R)1};  // the dummy member
+    auto stage = [&](int j, int id) {
+        sW[j] = p.W[id];
+        if constexpr (GEO) sC[j] = p.cen[id];
+    };
+    for (int i = t + NT; i < p.hfix; i += NT) stage(TILE + i, p.halo[(size_t)tile * p.hfix + i]);
+    for (int i = m0 + t; i < m1; i += NT) stage(TILE + p.hfix + i - m0, p.halo_more[i]);
     for (int i = t + NT; i < n16; i += NT) stDst[i] = stSrc[i];
     __syncthreads();
     if (!inb) return;  // the four lanes of a cell leave together
     const R* sWr = reinterpret_cast<const R*>(sW);
 
+    // the cell's member ids, eight to a 16-byte word; its compact neighbours
+    // (the cell itself where it has fewer than four)
+    const uint4* row = reinterpret_cast<const uint4*>(sRows + lc * SW);
+    const uint4 row0 = row[0];
+    const int nb[4] = {C > 0 ? (int)(row0.x & 0xffffu) : lc, C > 1 ? (int)(row0.x >> 16) : lc,
+                       C > 2 ? (int)(row0.y & 0xffffu) : lc, C > 3 ? (int)(row0.y >> 16) : lc};
+    const int nbl = (k & 2) ? ((k & 1) ? nb[3] : nb[2]) : ((k & 1) ? nb[1] : nb[0]);  // across lane k's slot
+
     // the temperature range over the compact stencil selects the branch
     R TMax = sWr[4 * lc + 3], TMin = TMax;
-    for (int i = 0; i < C; ++i) {
-        const R Tj = sWr[4 * sSt[sell(lc, i, maxS)] + 3];
-        TMax = fmax(Tj, TMax);
-        TMin = fmin(Tj, TMin);
+    {
+        R Tj[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) Tj[i] = sWr[4 * nb[i] + 3];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            TMax = fmax(Tj[i], TMax);
+            TMin = fmin(Tj[i], TMin);
+        }
+    }
+    double ex = 0.0, ey = 0.0;  // GEO: compact neighbour - cell centre of lane k's slot
+    if constexpr (GEO) {
+        // the host layout's expressions (face offset d, neighbour offset e):
+        // from the neighbour side the cell is seen shifted, from the owner's
+        // the neighbour; no shift enters at a boundary face
+        const double2 cc = sC[lc], cn = sC[nbl];
+        const double ax = live && isNei ? cc.x + fs.x : cc.x, ay = live && isNei ? cc.y + fs.y : cc.y;
+        const double bx = live && !isNei ? cn.x + fs.x : cn.x, by = live && !isNei ? cn.y + fs.y : cn.y;
+        if (has) {
+            d = v2{fc.x - ax, fc.y - ay};
+            ex = bx - ax;
+            ey = by - ay;
+        }
+        // k_lsq's sums over the compact slots in order, then lane k's weight;
+        // a lane without a slot adds 0 * 0
+        double Sxx = 0.0, Sxy = 0.0, Syy = 0.0;
+        const double qx[4] = {quad_bcast<0>(ex), quad_bcast<1>(ex), quad_bcast<2>(ex), quad_bcast<3>(ex)};
+        const double qy[4] = {quad_bcast<0>(ey), quad_bcast<1>(ey), quad_bcast<2>(ey), quad_bcast<3>(ey)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            Sxx += qx[i] * qx[i];
+            Sxy += qx[i] * qy[i];
+            Syy += qy[i] * qy[i];
+        }
+        const double det = Sxx * Syy - Sxy * Sxy;
+        const v2 m = v2{(Syy * ex - Sxy * ey) / det, (-Sxy * ex + Sxx * ey) / det};
+        if (has) Mk = m;
     }
     // Lane k forms variable k's least-squares gradient and compact-stencil
     // extrema (the reference's per-variable sums, in the same order; the
     // extrema are exact) and stores the gradient; the group then shares them.
     // The full path does this after its RBF sums, so that fewer values are
-    // live while the coefficients are in registers.
-    const int isNei = sf < 0;
-    const int f = (sf < 0 ? -sf : sf) - 1;
-    const bool live = k < C && f < nf;
-    double ex = 0.0, ey = 0.0;  // GEO: compact neighbour - cell centre of lane k's slot
-    if constexpr (GEO) {
-        // the host layout's expressions (face offset d, neighbour offset e)
-        if (k < C) {
-            const double2 cc = sC[lc];
-            const double2 cn = sC[sSt[sell(lc, k, maxS)]];
-            if (f < nf && !isNei) {
-                d = v2{fc.x - cc.x, fc.y - cc.y};
-                ex = (cn.x + fs.x) - cc.x;
-                ey = (cn.y + fs.y) - cc.y;
-            } else if (f < nf) {
-                const double xn = cc.x + fs.x, yn = cc.y + fs.y;
-                d = v2{fc.x - xn, fc.y - yn};
-                ex = cn.x - xn;
-                ey = cn.y - yn;
-            } else {
-                d = v2{fc.x - cc.x, fc.y - cc.y};
-                ex = cn.x - cc.x;
-                ey = cn.y - cc.y;
-            }
-        }
-        // k_lsq's sums over the compact slots in order, then lane k's weight
-        double Sxx = 0.0, Sxy = 0.0, Syy = 0.0;
-        const double bx[4] = {quad_bcast<0>(ex), quad_bcast<1>(ex), quad_bcast<2>(ex), quad_bcast<3>(ex)};
-        const double by[4] = {quad_bcast<0>(ey), quad_bcast<1>(ey), quad_bcast<2>(ey), quad_bcast<3>(ey)};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (i < C) {
-                Sxx += bx[i] * bx[i];
-                Sxy += bx[i] * by[i];
-                Syy += by[i] * by[i];
-            }
-        if (k < C)
-            Mk = v2{(Syy * ex - Sxy * ey) / (Sxx * Syy - Sxy * Sxy), (-Sxy * ex + Sxx * ey) / (Sxx * Syy - Sxy * Sxy)};
-    }
+    // live while the coefficients are in registers.  A missing neighbour adds
+    // 0 * 0, which leaves the sums (never -0) as they are.
     R gxk = 0, gyk = 0, mxk = 0, mnk = 0;
     auto gradient = [&]() {
         const R wck = sWr[4 * lc + k];
         mxk = wck;
         mnk = wck;
-        if constexpr (GEO) {
-            // every slot's weight from its lane, in slot order
-            const double mx[4] = {quad_bcast<0>(Mk.x), quad_bcast<1>(Mk.x), quad_bcast<2>(Mk.x), quad_bcast<3>(Mk.x)};
-            const double my[4] = {quad_bcast<0>(Mk.y), quad_bcast<1>(Mk.y), quad_bcast<2>(Mk.y), quad_bcast<3>(Mk.y)};
+        R cj[4];
+        v2 M[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (i < C) {
-                    const R cj = sWr[4 * sSt[sell(lc, i, maxS)] + k];
-                    const R dphi = cj - wck;
-                    gxk += mx[i] * dphi;
-                    gyk += my[i] * dphi;
-                    mxk = fmax(cj, mxk);
-                    mnk = fmin(cj, mnk);
-                }
-        } else {
-            for (int i = 0; i < C; ++i) {
-                const v2 M = sM[4 * lc + i];
-                const R cj = sWr[4 * sSt[sell(lc, i, maxS)] + k];
-                const R dphi = cj - wck;
-                gxk += M.x * dphi;
-                gyk += M.y * dphi;
-                mxk = fmax(cj, mxk);
-                mnk = fmin(cj, mnk);
-            }
+        for (int i = 0; i < 4; ++i) {
+            cj[i] = sWr[4 * nb[i] + k];
+            if constexpr (!GEO) M[i] = sM[4 * lc + i];
+        }
+        if constexpr (GEO) {  // every slot's weight from its lane
+            M[0] = v2{quad_bcast<0>(Mk.x), quad_bcast<0>(Mk.y)};
+            M[1] = v2{quad_bcast<1>(Mk.x), quad_bcast<1>(Mk.y)};
+            M[2] = v2{quad_bcast<2>(Mk.x), quad_bcast<2>(Mk.y)};
+            M[3] = v2{quad_bcast<3>(Mk.x), quad_bcast<3>(Mk.y)};
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const R dphi = i < C ? cj[i] - wck : (R)0;
+            gxk += M[i].x * dphi;
+            gyk += M[i].y * dphi;
+            mxk = fmax(cj[i], mxk);
+            mnk = fmin(cj[i], mnk);
         }
         v2* g = k == 0 ? p.gp : k == 1 ? p.gu : k == 2 ? p.gv : p.gT;
         g[c] = v2{gxk, gyk};
@@ -609,20 +650,13 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     if (k == 0) p.flat_prev[c] = flat;
     // Full path not foreseen: every RBF coefficient of the face and its centre
     // distance are requested now, at once (one memory round trip).
-    if (!flat && live && !early) {
-        if constexpr (!GEO) deltaR = p.slot_dr[sell(c, k, maxC)];
-#pragma unroll
-        for (int i = 0; i <= kMaxSten; ++i)
-            if (i <= S) cf[i] = a[(size_t)i * 64];
-    }
+    const bool late = !flat && live && !early;
+    if (__any(late)) load_coefficients(late);
     if constexpr (GEO) {
         if (!flat && live) deltaR = afar_hypot(ex, ey);  // k_lsq's centre distance
     }
     const R dx = d.x, dy = d.y;
-    R fraction = 0;
-    if (!flat && live) fraction = sqrt(dx * dx + dy * dy) / deltaR;
     const v4 wc = sW[lc];
-
     if (flat) {
         gradient();
         const R gpx = quad_bcast<0>(gxk), gpy = quad_bcast<0>(gyk), guxx = quad_bcast<1>(gxk),
@@ -657,22 +691,27 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
         return;
     }
 
-    R pf = 0, uxf = 0, uyf = 0, Tf = 0;
-    if (live) {
-        R coef = cf[0];
-        pf = coef * wc.x;
-        uxf = coef * wc.y;
-        uyf = coef * wc.z;
-        Tf = coef * wc.w;
+    // RBF sums, members four at a time up to the wavefront's longest stencil:
+    // the states of a round are requested together, and a cell that has no
+    // further members adds -0.0 * 1.
+    R pf = cf[0] * wc.x, uxf = cf[0] * wc.y, uyf = cf[0] * wc.z, Tf = cf[0] * wc.w;
+    {
+        const int rows = wave_max32(S, live);
+        uint4 ids = row0;
 #pragma unroll
-        for (int ci = 0; ci < kMaxSten; ++ci) {
-            if (ci < S) {
-                const v4 wj = sW[sSt[sell(lc, ci, maxS)]];
-                coef = cf[ci + 1];
-                pf += coef * wj.x;
-                uxf += coef * wj.y;
-                uyf += coef * wj.z;
-                Tf += coef * wj.w;
+        for (int j = 0; j < MS; j += 2) {
+            if (j < rows) {
+                if (j == 8 || j == 16) ids = row[j / 8];
+                const unsigned w2 = (j & 4) ? ((j & 2) ? ids.w : ids.z) : ((j & 2) ? ids.y : ids.x);
+                const v4 w4[2] = {sW[w2 & 0xffffu], sW[w2 >> 16]};
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const R coef = cf[j + i + 1];
+                    pf += coef * w4[i].x;
+                    uxf += coef * w4[i].y;
+                    uyf += coef * w4[i].z;
+                    Tf += coef * w4[i].w;
+                }
             }
         }
     }
@@ -688,9 +727,9 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     int faceNotTrouble = 1;
     if (live) {
         const R rP = fabs(pMax - pMin), rUx = fabs(uxMax - uxMin), rUy = fabs(uyMax - uyMin), rT = fabs(TMax - TMin);
-        const int nbl = sSt[sell(lc, k, maxS)];
         v4 o;
         R phif;
+        const R fraction = sqrt(dx * dx + dy * dy) / deltaR;
         limiter_process(limP, phif, wc.x, pMax, pMin, gpx, gpy, dx, dy);
         o.x = (R)(rP >= K<R>::SMALL) * pf + (R)(rP < K<R>::SMALL) * phif;
         smoothness = fmax(smoothness, fabs(((R)1 - fraction) * wc.x + fraction * sW[nbl].x - phif) / deltaR +
@@ -707,11 +746,11 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
         // or the unlimited linear state where the compact range is flat
         if constexpr (GP)
         for (int g = 0; g < p.ngp; ++g) {
-            const R* ag = p.rbf_gp + sell(c, (g * maxC + k) * (maxS + 1), p.ngp * KR);
+            const R* ag = p.rbf_gp + sell(c, (g * maxC + k) * (p.maxS + 1), p.ngp * KR);
             R cg = ag[0];
             R pg = cg * wc.x, uxg = cg * wc.y, uyg = cg * wc.z, Tg = cg * wc.w;
             for (int ci = 0; ci < S; ++ci) {
-                const v4 wj = sW[sSt[sell(lc, ci, maxS)]];
+                const v4 wj = sW[sRows[lc * SW + ci]];
                 cg = ag[(size_t)(ci + 1) * 64];
                 pg += cg * wj.x;
                 uxg += cg * wj.y;
@@ -791,14 +830,13 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
     int sfs[PF];
 #pragma unroll
     for (int fi = 0; fi < PF; ++fi) sfs[fi] = fi < maxC ? p.slot_face[sell(cc, fi, maxC)] : 0;
-    const int hb = p.halo_ptr[tile], hn = p.halo_ptr[tile + 1] - hb;
-    const int wpt = TILE >> 6;
-    const int nw = min(wpt, ((p.nc + 63) >> 6) - tile * wpt);
-    const int n16 = nw * maxS * 8;
-    const uint4* stSrc = reinterpret_cast<const uint4*>(p.sten + (size_t)tile * wpt * maxS * 64);
-    const int hmax = hn > 0 ? hn - 1 : 0;  // a tile without halo reads its first id harmlessly
-    const unsigned hid0 = (unsigned)p.halo[hb + min(tid, hmax)];
-    const unsigned hid1 = (unsigned)p.halo[hb + min(tid + TILE, hmax)];
+    const int n16 = sten_words(tile, TILE, p.nc, p.stenW);
+    const uint4* stSrc = reinterpret_cast<const uint4*>(p.sten + (size_t)tile * TILE * p.stenW);
+    const int hn = p.hfix;
+    const int32_t* hrow = p.halo + (size_t)tile * hn;
+    const unsigned hid0 = (unsigned)hrow[min(tid, hn - 1)];
+    const unsigned hid1 = (unsigned)hrow[min(tid + TILE, hn - 1)];
+    const int m0 = p.more_ptr[tile], m1 = p.more_ptr[tile + 1];
     const int8_t hs0 = p.smooth[hid0];
     const int8_t hs1 = p.smooth[hid1];
     // A face's test counts only in a limited cell (the limiter condition, or
@@ -826,11 +864,14 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
     if (tid < hn) sS[TILE + tid] = hs0;
     if (tid + TILE < hn) sS[2 * TILE + tid] = hs1;
     int flagged = (inb && own != 0) || (tid < hn && hs0 != 0) || (tid + TILE < hn && hs1 != 0);
-    for (int i = tid + 2 * TILE; i < hn; i += TILE) {
-        const int8_t h = p.smooth[p.halo[hb + i]];
-        sS[TILE + i] = h;
+    auto stage = [&](int j, int id) {
+        const int8_t h = p.smooth[id];
+        sS[j] = h;
         flagged |= h != 0;
-    }
+    };
+    for (int i = tid + 2 * TILE; i < hn; i += TILE) stage(TILE + i, hrow[i]);
+    for (int i = m0 + tid; i < m1; i += TILE) stage(TILE + hn + i - m0, p.halo_more[i]);
+    if (tid == 0) sS[TILE + p.hcap] = 0;  // the dummy member's flag
     int8_t shockType = own;
     int8_t shockTypeExt = own;
     // block-uniform: one wavefront's vote, or a workgroup reduction
@@ -846,11 +887,19 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
         for (int i = tid + 3 * TILE; i < n16; i += TILE) stDst[i] = stSrc[i];
         __syncthreads();
         if (inb) {
-            for (int ci = 0; ci < C; ++ci) {
-                shockType += sS[sSt[sell(tid, ci, maxS)]];
-                shockTypeExt = shockType;
+            // eight members to a 16-byte word of the cell's row; past its
+            // stencil the row names the dummy member, whose flag is 0
+            const uint4* row = reinterpret_cast<const uint4*>(sSt + tid * p.stenW);
+            for (int ci = 0; ci < S; ci += 8) {
+                const uint4 q = row[ci >> 3];
+                const unsigned ids[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int8_t h = sS[(i & 1) ? ids[i >> 1] >> 16 : ids[i >> 1] & 0xffffu];
+                    if (ci + i < C) shockType += h;
+                    shockTypeExt += h;
+                }
             }
-            for (int ci = C; ci < S; ++ci) shockTypeExt += sS[sSt[sell(tid, ci, maxS)]];
         }
     }
     if (!inb) return;
@@ -1440,14 +1489,24 @@ void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, hipStream
     hipLaunchKernelGGL(k_cfl<R>, dim3(nt), dim3(256), 0, s, p, Rg, Cv, CFL, chunk);
 }
 
+template <typename R, bool GP, int MS>
+void launch_reconstruct_q(const DevPtrs<R>& p, int nb, int tile, size_t lds, hipStream_t s) {
+    switch (tile) {
+        case 64: hipLaunchKernelGGL((k_reconstruct_q<R, 64, GP, MS>), dim3(nb), dim3(256), lds, s, p); break;
+        case 128: hipLaunchKernelGGL((k_reconstruct_q<R, 128, GP, MS>), dim3(nb), dim3(512), lds, s, p); break;
+        default: hipLaunchKernelGGL((k_reconstruct_q<R, 256, GP, MS>), dim3(nb), dim3(1024), lds, s, p); break;
+    }
+}
+
 template <typename R, bool GP>
 void launch_reconstruct_t(const DevPtrs<R>& p, int nb, int tile, size_t lds, hipStream_t s, int lanes) {
     if (lanes == 4) {
-        switch (tile) {
-            case 64: hipLaunchKernelGGL((k_reconstruct_q<R, 64, GP>), dim3(nb), dim3(256), lds, s, p); break;
-            case 128: hipLaunchKernelGGL((k_reconstruct_q<R, 128, GP>), dim3(nb), dim3(512), lds, s, p); break;
-            default: hipLaunchKernelGGL((k_reconstruct_q<R, 256, GP>), dim3(nb), dim3(1024), lds, s, p); break;
-        }
+        if (p.maxS <= 8)
+            launch_reconstruct_q<R, GP, 8>(p, nb, tile, lds, s);
+        else if (p.maxS <= 16)
+            launch_reconstruct_q<R, GP, 16>(p, nb, tile, lds, s);
+        else
+            launch_reconstruct_q<R, GP, kMaxSten>(p, nb, tile, lds, s);
         return;
     }
     switch (tile) {
@@ -1520,12 +1579,16 @@ void launch_update(const DevPtrs<R>& p, double Rg, double gamma, double dt, cons
 template <typename R>
 hipError_t set_lds_limits(size_t lds) {
     hipError_t e = hipSuccess;
-    const void* fns[] = {(const void*)k_reconstruct<R, 64, false>,    (const void*)k_reconstruct<R, 128, false>,
-                         (const void*)k_reconstruct<R, 256, false>,   (const void*)k_reconstruct_q<R, 64, false>,
-                         (const void*)k_reconstruct_q<R, 128, false>, (const void*)k_reconstruct_q<R, 256, false>,
-                         (const void*)k_reconstruct<R, 64, true>,     (const void*)k_reconstruct<R, 128, true>,
-                         (const void*)k_reconstruct<R, 256, true>,    (const void*)k_reconstruct_q<R, 64, true>,
-                         (const void*)k_reconstruct_q<R, 128, true>,  (const void*)k_reconstruct_q<R, 256, true>};
+#define AFAR_Q_KERNELS(GP, MS)                                                                     \
+    (const void*)k_reconstruct_q<R, 64, GP, MS>, (const void*)k_reconstruct_q<R, 128, GP, MS>, \
+        (const void*)k_reconstruct_q<R, 256, GP, MS>
+    const void* fns[] = {(const void*)k_reconstruct<R, 64, false>,  (const void*)k_reconstruct<R, 128, false>,
+                         (const void*)k_reconstruct<R, 256, false>, (const void*)k_reconstruct<R, 64, true>,
+                         (const void*)k_reconstruct<R, 128, true>,  (const void*)k_reconstruct<R, 256, true>,
+                         AFAR_Q_KERNELS(false, 8),                  AFAR_Q_KERNELS(false, 16),
+                         AFAR_Q_KERNELS(false, kMaxSten),           AFAR_Q_KERNELS(true, 8),
+                         AFAR_Q_KERNELS(true, 16),                  AFAR_Q_KERNELS(true, kMaxSten)};
+#undef AFAR_Q_KERNELS
     for (const void* fn : fns) {
         // the dynamic limit plus the kernel's static LDS may not exceed the block limit
         hipFuncAttributes attr;

@@ -472,15 +472,19 @@ DevLayout make_dev_layout(const RefArrays& ra, int tile) {
     const int KR = maxC * (maxS + 1);
     L.scnt = ra.stencilSize;
     L.ccnt = ra.compactStencilSize;
-    L.sten.assign((size_t)L.nwaves * std::max(maxS, 1) * 64, 0);
+    L.stenW = std::max(8, (maxS + 7) & ~7);
+    L.sten.assign((size_t)L.nwaves * 64 * L.stenW, 0);
     L.slot_face.assign(nslot, 0);
     L.slot_d.assign(2 * nslot, 0.0);
     L.slot_e.assign(2 * nslot, 0.0);
-    L.rbf.assign((size_t)L.nwaves * KR * 64, 0.0);
+    // Rows past a cell's stencil hold -0.0 and their ids name a dummy member of
+    // state 1: the terms -0.0 * 1 that a whole wavefront's loop adds for a cell
+    // of a shorter stencil leave every sum as it is.
+    L.rbf.assign((size_t)L.nwaves * KR * 64, -0.0);
     L.ngp = ra.ngp;
     L.gpw = ra.GPW;
     L.fgd = ra.GPD;
-    L.rbf_gp.assign((size_t)L.nwaves * ra.ngp * KR * 64, 0.0);
+    L.rbf_gp.assign((size_t)L.nwaves * ra.ngp * KR * 64, -0.0);
     L.vol = ra.cellVolume;
     const double* CELL = ra.CELL.data();
     const double* FACE = ra.FACE.data();
@@ -511,20 +515,38 @@ DevLayout make_dev_layout(const RefArrays& ra, int tile) {
                             local = it->second;
                         }
                     }
-                    if (local > 65535) overflow[t] = 1;
-                    L.sten[L.sell(c, i, maxS)] = (uint16_t)local;
+                    if (local > 65534) overflow[t] = 1;
+                    L.sten[(size_t)c * L.stenW + i] = (uint16_t)local;
                 }
         }
     });
     for (int t = 0; t < L.ntiles; ++t)
         if (overflow[t]) throw Error(3, "Too large local block stencil size (LDS ids exceed 16 bits)");
-    L.halo_ptr.assign(L.ntiles + 1, 0);
+    std::vector<int> count(L.ntiles);
     for (int t = 0; t < L.ntiles; ++t) {
-        L.halo_ptr[t + 1] = L.halo_ptr[t] + (int32_t)halos[t].size();
-        L.maxHalo = std::max(L.maxHalo, (int)halos[t].size());
+        count[t] = (int)halos[t].size();
+        L.maxHalo = std::max(L.maxHalo, count[t]);
     }
-    L.halo.resize(L.halo_ptr[L.ntiles]);
-    for (int t = 0; t < L.ntiles; ++t) std::copy(halos[t].begin(), halos[t].end(), L.halo.begin() + L.halo_ptr[t]);
+    // the row width that holds all but one in fifty of the lists
+    if (L.ntiles) {
+        const int q = std::min(L.ntiles - 1, L.ntiles * 49 / 50);
+        std::nth_element(count.begin(), count.begin() + q, count.end());
+        L.hfix = std::max(1, std::min((count[q] + 3) & ~3, L.maxHalo));
+    }
+    L.hcap = std::max(L.hfix, L.maxHalo);
+    if (L.tile + L.hcap > 65535) throw Error(3, "Too large local block stencil size (LDS ids exceed 16 bits)");
+    L.halo.resize((size_t)L.ntiles * L.hfix);
+    L.more_ptr.assign(L.ntiles + 1, 0);
+    L.halo_more.clear();
+    for (int t = 0; t < L.ntiles; ++t) {
+        const auto& h = halos[t];
+        for (int i = 0; i < L.hfix; ++i) L.halo[(size_t)t * L.hfix + i] = i < (int)h.size() ? h[i] : t * tile;
+        for (int i = L.hfix; i < (int)h.size(); ++i) L.halo_more.push_back(h[i]);
+        L.more_ptr[t + 1] = (int32_t)L.halo_more.size();
+    }
+    for (int c = 0; c < L.nwaves * 64; ++c)
+        for (int i = c < nc ? ra.stencilSize[c] : 0; i < L.stenW; ++i)
+            L.sten[(size_t)c * L.stenW + i] = (uint16_t)(tile + L.hcap);
 
     // slots: face ids, geometry, RBF coefficients
     parallel_for(nc, [&](int64_t c0, int64_t c1) {

@@ -59,12 +59,19 @@ struct DevLayout {
     int nwaves = 0, ntiles = 0, maxHalo = 0;
     // per cell
     std::vector<uint8_t> scnt, ccnt;      // nc
-    std::vector<uint16_t> sten;           // nwaves*maxS*64, LDS-local ids
+    int stenW = 8;                        // ids per row of sten: maxS rounded up to whole 16-byte words
+    std::vector<uint16_t> sten;           // nwaves*64*stenW, one row per cell: LDS-local ids, then the tile's
+                                          // dummy member (tile + hcap)
     std::vector<int32_t> slot_face;       // nwaves*maxC*64, +-(f+1), 0 = padding
     std::vector<double> slot_d;           // 2 per slot: face centre - cell centre
     std::vector<double> slot_e;           // 2 per slot: compact neighbour - cell centre
-    std::vector<double> rbf;              // nwaves*maxC*(maxS+1)*64
-    std::vector<int32_t> halo_ptr, halo;  // ntiles+1, global ids of halo members
+    std::vector<double> rbf;              // nwaves*maxC*(maxS+1)*64, padding -0.0
+    // Global ids of a tile's halo members: the first hfix in a row of fixed
+    // width (a short list repeats the tile's first cell), the rest of the few
+    // longer lists in halo_more[more_ptr[tile] .. more_ptr[tile + 1]).  hcap:
+    // the larger of hfix and the longest list.
+    int hfix = 1, hcap = 1;
+    std::vector<int32_t> halo, more_ptr, halo_more;
     // per internal face
     std::vector<int32_t> fcell;           // 2*nf: own, nei
     std::vector<double> fgeo;             // 8*nf: Sfx, Sfy, magSf, deltaR, dxo, dyo, dxn, dyn

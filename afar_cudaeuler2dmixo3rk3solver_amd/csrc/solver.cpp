@@ -63,6 +63,41 @@ struct StreamHolder {
     }
 };
 
+// Threads per cell of the reconstruction: four measured fastest at 64 and 128-cell tiles.
+int recon_lanes(const DevLayout& L, const SolverConfig& cfg) {
+    return cfg.reconLanes != 0 ? cfg.reconLanes : L.maxC > 4 ? 1 : 4;
+}
+
+// LDS of the reconstruction: the states of the tile and of `halo` more, rows of
+// `ids` stencil ids; the four-lane kernel also stages the tile's least-squares
+// weights (FP64 at the face centre: the tile's and halo's centres in their place).
+size_t recon_lds(const DevLayout& L, const SolverConfig& cfg, size_t halo, size_t ids) {
+    const size_t w = cfg.precision == 1 ? sizeof(float) : sizeof(double), nst = L.tile + halo;
+    size_t n = nst * 4 * w + (size_t)L.tile * ids * sizeof(uint16_t);
+    if (recon_lanes(L, cfg) == 4)
+        n = ((n + 15) & ~(size_t)15) + std::max((size_t)L.tile * 8 * w, w == 8 ? nst * 16 : (size_t)0);
+    return n;
+}
+
+size_t lds_limit() {
+    int dev = 0;
+    check_hip(hipGetDevice(&dev), "hipGetDevice");
+    hipDeviceProp_t prop;
+    check_hip(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
+    return prop.sharedMemPerBlock;
+}
+
+// The device layout in tiles of cfg.tile cells.  Its dummy member and whole
+// 16-byte rows of ids take up to 14 bytes a cell and 48 more than the bare
+// states and ids: a tile that only they push over the LDS limit is halved.
+DevLayout solver_layout(const RefArrays& ra, const SolverConfig& cfg) {
+    DevLayout L = make_dev_layout(ra, cfg.tile);
+    const size_t cap = lds_limit();
+    if (cfg.tile > 64 && recon_lds(L, cfg, L.hcap + 1, L.stenW) > cap && recon_lds(L, cfg, L.maxHalo, L.maxS) <= cap)
+        L = make_dev_layout(ra, cfg.tile / 2);
+    return L;
+}
+
 template <typename R>
 class SolverImpl final : public DeviceSolver {
     using v4 = typename VT<R>::v4;
@@ -94,27 +129,15 @@ class SolverImpl final : public DeviceSolver {
         check_hip(hipEventCreate(&ev0_), "hipEventCreate");
         check_hip(hipEventCreate(&ev1_), "hipEventCreate");
         for (hipEvent_t& e : evq_) check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-        // LDS of the reconstruction: tile + halo states, then the tile's stencil ids
-        lds_recon_ = (size_t)(L_.tile + L_.maxHalo) * sizeof(v4) + (size_t)L_.tile * L_.maxS * sizeof(uint16_t);
-        lds_m_off_ = (lds_recon_ + 15) & ~(size_t)15;
         if (cfg.reconLanes == 4 && L_.maxC > 4) throw Error(1, "reconLanes 4 needs cells with at most four faces");
-        if (cfg.reconLanes != 0)
-            lanes_ = cfg.reconLanes;
-        else
-            lanes_ = L_.maxC > 4 ? 1 : 4;  // four lanes measured fastest at 64 and 128-cell tiles
-        // the four-lane kernel also stages the tile's least-squares weights
-        // (FP64 at the face centre: the tile's and halo's centres in their place)
-        if (lanes_ == 4)
-            lds_recon_ = lds_m_off_ + std::max((size_t)L_.tile * 4 * sizeof(v2),
-                                               sizeof(R) == 8 ? (size_t)(L_.tile + L_.maxHalo) * 16 : (size_t)0);
+        lanes_ = recon_lanes(L_, cfg);
+        const size_t nst = (size_t)L_.tile + L_.hcap + 1, sten_bytes = (size_t)L_.tile * L_.stenW * sizeof(uint16_t);
+        lds_m_off_ = (nst * sizeof(v4) + sten_bytes + 15) & ~(size_t)15;
+        lds_recon_ = recon_lds(L_, cfg, L_.hcap + 1, L_.stenW);
         // BVD: the tile's and halo's smoothness flags, then the stencil ids
-        lds_bvd_sten_off_ = ((size_t)(L_.tile + L_.maxHalo) + 15) & ~(size_t)15;
-        lds_bvd_ = lds_bvd_sten_off_ + (size_t)L_.tile * L_.maxS * sizeof(uint16_t);
-        int dev = 0;
-        check_hip(hipGetDevice(&dev), "hipGetDevice");
-        hipDeviceProp_t prop;
-        check_hip(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
-        size_t lds_cap = prop.sharedMemPerBlock;
+        lds_bvd_sten_off_ = (nst + 15) & ~(size_t)15;
+        lds_bvd_ = lds_bvd_sten_off_ + sten_bytes;
+        const size_t lds_cap = lds_limit();
         if (lds_recon_ > lds_cap)
             throw Error(3, "Too large local block stencil size: reconstruct needs " +
                                std::to_string(lds_recon_) + " bytes of LDS, the device allows " +
@@ -617,7 +640,10 @@ class SolverImpl final : public DeviceSolver {
         P_.maxS = L_.maxS;
         P_.maxC = L_.maxC;
         P_.ntiles = L_.ntiles;
-        P_.lds_sten_off = (int)((size_t)(L_.tile + L_.maxHalo) * sizeof(v4));
+        P_.lds_sten_off = (int)((size_t)(L_.tile + L_.hcap + 1) * sizeof(v4));
+        P_.stenW = L_.stenW;
+        P_.hfix = L_.hfix;
+        P_.hcap = L_.hcap;
         P_.lds_m_off = (int)lds_m_off_;
         P_.lds_bvd_sten_off = (int)lds_bvd_sten_off_;
         P_.boundaryFirstOrder = cfg_.boundaryFirstOrder;
@@ -660,14 +686,9 @@ class SolverImpl final : public DeviceSolver {
         dalloc(m_lsq, sizeof(v2) * nslot);
         P_.lsq = m_lsq.as<v2>();
         P_.rbf = put_as_R(m_rbf, L_.rbf.data(), L_.rbf.size());
-        P_.halo_ptr = put(m_halo_ptr, L_.halo_ptr.data(), L_.halo_ptr.size());
-        {
-            // one trailing id (cell 0) so that a tile without halo may read
-            // its first id unconditionally
-            std::vector<int32_t> halo(L_.halo.begin(), L_.halo.end());
-            halo.push_back(0);
-            P_.halo = put(m_halo, halo.data(), halo.size());
-        }
+        P_.halo = put(m_halo, L_.halo.data(), L_.halo.size());
+        P_.more_ptr = put(m_more_ptr, L_.more_ptr.data(), L_.more_ptr.size());
+        P_.halo_more = put(m_halo_more, L_.halo_more.data(), L_.halo_more.size());
         P_.fcell = reinterpret_cast<const int2*>(put(m_fcell, L_.fcell.data(), 2 * nf));
         P_.fgeo = reinterpret_cast<const double4*>(put(m_fgeo, L_.fgeo.data(), 8 * nf));
         // Cell and face centres (and periodic shifts): the FP64 four-lane
@@ -789,7 +810,7 @@ class SolverImpl final : public DeviceSolver {
         // the host keeps only what set_conserved needs (state, faces, boundary table)
         release_host(ra_.RBFbasis, ra_.RBFgp, ra_.stencil, ra_.cellFaces, ra_.neighbour, ra_.GPD);
         release_host(L_.rbf, L_.rbf_gp, L_.slot_d, L_.slot_e, L_.fgeo, L_.fgd);
-        release_host(L_.sten, L_.slot_face, L_.fcell, L_.halo);
+        release_host(L_.sten, L_.slot_face, L_.fcell, L_.halo, L_.halo_more);
     }
 
     template <typename... V> static void release_host(V&... v) { ((void)std::decay_t<V>().swap(v), ...); }
@@ -813,7 +834,7 @@ class SolverImpl final : public DeviceSolver {
     size_t lds_recon_ = 0, lds_bvd_ = 0, lds_m_off_ = 0, lds_bvd_sten_off_ = 0;
     int lanes_ = 1;  // threads per cell of the reconstruction kernel
     DevMem m_W, m_U, m_Uold, m_vol, m_gp, m_gu, m_gv, m_gT, m_lim, m_smooth, m_ftype, m_scnt, m_ccnt, m_sten,
-        m_slot_face, m_slot_d, m_slot_e, m_slot_dr, m_lsq, m_rbf, m_halo_ptr, m_halo, m_fcell, m_fgeo, m_fgeo32,
+        m_slot_face, m_slot_d, m_slot_e, m_slot_dr, m_lsq, m_rbf, m_halo, m_more_ptr, m_halo_more, m_fcell, m_fgeo, m_fgeo32,
         m_fv, m_fvp, m_fvu, m_fvv, m_flux, m_flux32, m_bcell, m_blabel, m_bgeo, m_bval, m_dt, m_fvT, m_cinst, m_finst, m_tctl, m_res,
         m_rbf_gp, m_fgd, m_fvg, m_flat_prev, m_tlim, m_tTVD, m_cen, m_fcen, m_fshift, m_fsf, m_fmag;
 };
@@ -969,7 +990,7 @@ std::unique_ptr<DeviceSolver> make_device_solver(const RefArrays& ra, const Solv
     // overlap in it; the lock covers the device allocation and upload
     if (cfg.cellOrder == 1) {
         RefArrays copy = ra;
-        DevLayout L = make_dev_layout(copy, cfg.tile);
+        DevLayout L = solver_layout(copy, cfg);
         std::lock_guard<std::mutex> lk(runtime_mutex());
         return make_impl(std::move(copy), std::move(L), cfg, bi);
     }
@@ -986,7 +1007,7 @@ std::unique_ptr<DeviceSolver> make_device_solver(const RefArrays& ra, const Solv
     std::unique_ptr<DeviceSolver> in;
     {
         RefArrays rl = relabel(ra, r);
-        DevLayout L = make_dev_layout(rl, cfg.tile);
+        DevLayout L = solver_layout(rl, cfg);
         std::lock_guard<std::mutex> lk(runtime_mutex());
         in = make_impl(std::move(rl), std::move(L), cfg, bi);
     }
