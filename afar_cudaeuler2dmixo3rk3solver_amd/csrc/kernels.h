@@ -74,7 +74,7 @@ struct DevPtrs {
     // 16-byte record.  The BVD test reads fvT alone.
     typename VT<R>::v4* fv;
     R *fvp, *fvu, *fvv, *fvT;
-    R* tTVD;                   // 2*nf the BVD test's limited linear face temperature of that side's cell,
+    R* tTVD;                   // sliced ELL, the BVD test's limited linear temperature on the cell's face,
                                // Tc + BJ(raw T limiter) * (grad T . d), formed by the reconstruction
     int8_t* tlim;              // nc: BJ(raw T limiter) < VALID_LIM_FACTOR (the BVD test's limiter condition)
     // extension (faceQuadrature): flux at ngp points per internal face

@@ -744,7 +744,7 @@ class SolverImpl final : public DeviceSolver {
         }
         dalloc(m_fvT, sizeof(R) * 2 * nf);
         P_.fvT = m_fvT.as<R>();
-        dalloc(m_tTVD, sizeof(R) * 2 * nf);
+        dalloc(m_tTVD, sizeof(R) * nslot);
         P_.tTVD = m_tTVD.as<R>();
         P_.ngp = L_.ngp;
         if (L_.ngp > 4) throw Error(3, "more than four flux quadrature points");
