@@ -34,10 +34,16 @@ struct DevPtrs {
     double4* Uold;             // nc
     const double* vol;         // nc
     typename VT<R>::v2 *gp, *gu, *gv, *gT;  // nc: grad p; (dUx/dx, dUx/dy); (dUy/dx, dUy/dy); grad T
-    typename VT<R>::v4* lim;   // nc limiters p, Ux, Uy, T
+    typename VT<R>::v4* lim;   // nc limiters p, Ux, Uy, T, then one entry of ones
     int8_t* smooth;            // nc+nb smoothness flag (shockIndicator[2c])
     int8_t* ftype;             // nc final reconstruction type (shockIndicator[2c+1])
-    uint8_t* flat_prev;        // nc: the cell took the flat branch at the last reconstruction (load scheduling only)
+    uint8_t* flat_prev;        // nc: the cell took the flat branch at the last reconstruction
+    // nf pairs (own, nei), face-centre path: that side's cell is flat, so its
+    // face state is W + grad . d and its limiters 1; the face pass forms both
+    // and the reconstruction stores neither (storeFlat: it stores them too).
+    // Written only where a cell's branch changed.
+    uint8_t* fflat;
+    int storeFlat;
     const uint8_t* scnt;       // nc stencil size
     const uint8_t* ccnt;       // nc compact stencil size
     int stenW;                 // ids per row of sten, a multiple of 8

@@ -205,6 +205,18 @@ template <typename R> __device__ __forceinline__ R to_venkat(R y) {
     return fmin((y * y + y + K<R>::VSMALL) / (y * y + (R)0.5 + (R)0.5 * y + K<R>::VSMALL), (R)1);
 }
 
+// Whether the face pass forms a flat cell's face states and limiters (FP64 at
+// the face centre): the reconstruction then writes 24 B per face side and 32 B
+// per cell less, and the face pass reads 64 B per face and 32 B per cell less,
+// where the gas is uniform, as ahead of every wave.  1.5M cells, 60% of them on
+// the full path: reconstruct 219 -> 192 us, flux 118 -> 114, step 1265 -> 1172;
+// nine corner flows 525 -> 480; 45k and 157k corner quads 105 -> 100, 167 ->
+// 159; 20k 83.6 -> 83.0; with no flat cell 67.9 -> 68.2.  FP32-mixed has half
+// the bytes to save and was slower for it (740k cells 469 -> 480).
+template <typename R, bool GP> struct FormsFlat {
+    static constexpr bool value = sizeof(R) == 8 && !GP;
+};
+
 // GP: the flux-quadrature extension's point states (a separate instantiation,
 // so the reference path carries none of its registers)
 template <typename R, int TILE, bool GP>
@@ -267,8 +279,27 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
     }
 
     const int nf = p.nf;
-    if (fabs(TMax - TMin) < K<R>::VSMALL) {
-        p.lim[c] = v4{(R)1, (R)1, (R)1, (R)1};
+    // as in k_reconstruct_q: the cells whose face states and limiters the face pass forms
+    const bool flat = fabs(TMax - TMin) < K<R>::VSMALL;
+    bool skip = false;
+    if constexpr (FormsFlat<R, GP>::value) {
+        bool edge = false;
+        if (p.boundaryFirstOrder)
+            for (int fi = 0; fi < C; ++fi) edge = edge || abs(p.slot_face[sell(c, fi, maxC)]) - 1 >= nf;
+        skip = flat && !edge;
+        const bool wasFlat = p.flat_prev[c] != 0;
+        if (flat != wasFlat) {
+            p.flat_prev[c] = flat;
+            for (int fi = 0; fi < C; ++fi) {
+                const int sf = p.slot_face[sell(c, fi, maxC)];
+                const int f = (sf < 0 ? -sf : sf) - 1;
+                if (f < nf) p.fflat[2 * f + (sf < 0)] = skip;
+            }
+        }
+    }
+    if (flat) {
+        const bool store = !skip || p.storeFlat;
+        if (store) p.lim[c] = v4{(R)1, (R)1, (R)1, (R)1};
         const R lT = to_bj((R)1);  // the BVD test's limiter of this cell
         p.tlim[c] = lT < K<R>::VALID_LIM_FACTOR;
         for (int fi = 0; fi < C; ++fi) {
@@ -283,7 +314,10 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
             o.y = wc.y + guxx * dx + guyx * dy;
             o.z = wc.z + guxy * dx + guyy * dy;
             o.w = wc.w + gTx * dx + gTy * dy;
-            store_face_state(p, 2 * f + isNei, o);
+            if (store)
+                store_face_state(p, 2 * f + isNei, o);
+            else
+                p.fvT[2 * f + isNei] = o.w;
             p.tTVD[sell(c, fi, maxC)] = wc.w + lT * (gTx * dx + gTy * dy);
             if constexpr (GP)
                 for (int g = 0; g < p.ngp; ++g) {  // flux points (extension): the same linear state there
@@ -461,6 +495,7 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     // operations in their order, instead of reading 40 bytes of stored slot
     // data per slot; the weights are shared within the group by DPP.
     constexpr bool GEO = sizeof(R) == 8 && !GP;
+    constexpr bool FLAT = FormsFlat<R, GP>::value;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     v4* sW = reinterpret_cast<v4*>(smem_raw);
     uint16_t* sRows = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
@@ -655,7 +690,13 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     };
     const bool flat = fabs(TMax - TMin) < K<R>::VSMALL;
 
-    if (k == 0) (p.flat_prev + c0)[lc] = flat;
+    if (k == 0 && flat != (wasFlat != 0)) (p.flat_prev + c0)[lc] = flat;
+    // The face pass forms a flat cell's face states and limiters itself
+    // (DevPtrs::fflat); a first-order boundary cell's limiter is the BVD pass's.
+    bool edge = false;
+    if (FLAT && p.boundaryFirstOrder) edge = ((__ballot(has && !live) >> ((t & 63) & ~3)) & 0xF) != 0;
+    const bool skip = FLAT && flat && !edge;
+    if (FLAT && live && skip != (wasFlat && !edge)) p.fflat[2 * f + isNei] = skip;
     // Full path not foreseen: every RBF coefficient of the face and its centre
     // distance are requested now, at once (one memory round trip).
     const bool late = !flat && live && !early;
@@ -671,18 +712,23 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
                 guyx = quad_bcast<1>(gyk), guxy = quad_bcast<2>(gxk), guyy = quad_bcast<2>(gyk),
                 gTx = quad_bcast<3>(gxk), gTy = quad_bcast<3>(gyk);
         const R lT = to_bj((R)1);  // the BVD test's limiter of this cell
+        const bool store = !skip || p.storeFlat;
         if (k == 0) {
-            (p.lim + c0)[lc] = v4{(R)1, (R)1, (R)1, (R)1};
+            if (store) (p.lim + c0)[lc] = v4{(R)1, (R)1, (R)1, (R)1};
             (p.smooth + c0)[lc] = 0;
             (p.tlim + c0)[lc] = lT < K<R>::VALID_LIM_FACTOR;
         }
         if (live) {
             v4 o;
-            o.x = wc.x + gpx * dx + gpy * dy;
-            o.y = wc.y + guxx * dx + guyx * dy;
-            o.z = wc.z + guxy * dx + guyy * dy;
             o.w = wc.w + gTx * dx + gTy * dy;
-            store_face_state(p, 2 * f + isNei, o);
+            if (store) {
+                o.x = wc.x + gpx * dx + gpy * dy;
+                o.y = wc.y + guxx * dx + guyx * dy;
+                o.z = wc.z + guxy * dx + guyy * dy;
+                store_face_state(p, 2 * f + isNei, o);
+            } else {
+                p.fvT[2 * f + isNei] = o.w;
+            }
             slots(p.tTVD)[row_k] = wc.w + lT * (gTx * dx + gTy * dy);
             if constexpr (GP)
                 for (int g = 0; g < p.ngp; ++g) {  // flux points (extension): the same linear state there
@@ -1108,6 +1154,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
     DevPtrs<R> p, double Rgas, double Cv, double CFL) {
     using v4 = typename VT<R>::v4;
     using v2 = typename VT<R>::v2;
+    constexpr bool FLAT = FormsFlat<R, GP>::value;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const int i = tile * 256 + threadIdx.x;
     const int nf = p.nf;
@@ -1116,6 +1163,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
         const int f = i;
         const int2 oc = p.fcell[f];
         const int own = oc.x, nei = oc.y;
+        // sides whose face state and limiters are formed here (DevPtrs::fflat)
+        bool skL = false, skR = false;
+        if constexpr (FLAT) {
+            const uchar2 sk = reinterpret_cast<const uchar2*>(p.fflat)[f];
+            skL = sk.x != 0;
+            skR = sk.y != 0;
+        }
         double4 g0, g1;
         if constexpr (sizeof(R) == 4 && !DT) {  // the geometry as the float arithmetic uses it
             const float4 h0 = p.fgeo32[2 * f], h1 = p.fgeo32[2 * f + 1];
@@ -1148,16 +1202,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
         const R magSf = (R)g0.z, Sfx = (R)g0.x, Sfy = (R)g0.y;
         const R Rg = (R)Rgas;
         const v4 wL = p.W[own], wR = p.W[nei];
-        const v4 rL = p.lim[own], rR = p.lim[nei];
-        const int shL = to < 0, shR = tn < 0;
-        const v4 lL = face_limiters<R>(rL, shL);
-        const v4 lR = face_limiters<R>(rR, shR);
-        // face-centre O3 states of both sides
+        const v2 gpL = p.gp[own], gTL = p.gT[own];
+        const v2 gpR = p.gp[nei], gTR = p.gT[nei];
+        // Raw limiters and face-centre O3 states of both sides.  A flat side
+        // reads the entry of ones behind the cells' limiters, a face with two
+        // of them face 0's states: no branches, and no memory traffic.
+        const v4 rL = p.lim[FLAT && skL ? p.nc : own], rR = p.lim[FLAT && skR ? p.nc : nei];
         v4 fL0{}, fR0{};
         if constexpr (!GP) {
             if constexpr (sizeof(R) == 8) {  // one 2-vector per variable
-                const v2 sp = reinterpret_cast<const v2*>(p.fvp)[f], su = reinterpret_cast<const v2*>(p.fvu)[f];
-                const v2 sv = reinterpret_cast<const v2*>(p.fvv)[f], sT = reinterpret_cast<const v2*>(p.fvT)[f];
+                const int fr = skL && skR ? 0 : f;
+                const v2 sp = reinterpret_cast<const v2*>(p.fvp)[fr], su = reinterpret_cast<const v2*>(p.fvu)[fr];
+                const v2 sv = reinterpret_cast<const v2*>(p.fvv)[fr], sT = reinterpret_cast<const v2*>(p.fvT)[fr];
                 fL0 = v4{sp.x, su.x, sv.x, sT.x};
                 fR0 = v4{sp.y, su.y, sv.y, sT.y};
             } else {
@@ -1165,8 +1221,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
                 fR0 = p.fv[2 * f + 1];
             }
         }
-        const v2 gpL = p.gp[own], gTL = p.gT[own];
-        const v2 gpR = p.gp[nei], gTR = p.gT[nei];
+        if (DT) {
+            const double d = cfl_face_dt(g0, g1, wL, wR, Rgas, Cv, CFL);
+            dtf = d < dtf ? d : dtf;
+        }
+        const int shL = to < 0, shR = tn < 0;
+        const v4 lL = face_limiters<R>(rL, shL);
+        const v4 lR = face_limiters<R>(rR, shR);
         // The limited linear velocities enter the flux only on a TVD side: on
         // an O3 side they are blended with weight 0, which adds a zero to the
         // O3 velocity, so they change nothing unless that velocity is itself a
@@ -1174,20 +1235,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
         // only where they can matter (at the face centre).  A non-finite
         // velocity gradient beside a finite O3 state (a degenerate
         // least-squares stencil) would turn that blend into NaN in the
-        // reference; here it is not read.
+        // reference; here it is not read.  A flat cell's state is linear and
+        // takes them too; it is formed with the reconstruction's operations.
         v2 guL{}, gvL{}, guR{}, gvR{};
-        if (GP || isTVD_L || fL0.y == (R)0 || fL0.z == (R)0) {
+        if (GP || skL || isTVD_L || fL0.y == (R)0 || fL0.z == (R)0) {
             guL = p.gu[own];
             gvL = p.gv[own];
         }
-        if (GP || isTVD_R || fR0.y == (R)0 || fR0.z == (R)0) {
+        if (GP || skR || isTVD_R || fR0.y == (R)0 || fR0.z == (R)0) {
             guR = p.gu[nei];
             gvR = p.gv[nei];
         }
-        if (DT) {
-            const double d = cfl_face_dt(g0, g1, wL, wR, Rgas, Cv, CFL);
-            dtf = d < dtf ? d : dtf;
-        }
+        if (FLAT && skL)
+            fL0 = v4{wL.x + gpL.x * dxL + gpL.y * dyL, wL.y + guL.x * dxL + guL.y * dyL,
+                     wL.z + gvL.x * dxL + gvL.y * dyL, wL.w + gTL.x * dxL + gTL.y * dyL};
+        if (FLAT && skR)
+            fR0 = v4{wR.x + gpR.x * dxR + gpR.y * dyR, wR.y + guR.x * dxR + guR.y * dyR,
+                     wR.z + gvR.x * dxR + gvR.y * dyR, wR.w + gTR.x * dxR + gTR.y * dyR};
 
         // the flux of the two states reconstructed at a point with offsets
         // (dxL, dyL) from the owner and (dxR, dyR) from the neighbour; fL, fR

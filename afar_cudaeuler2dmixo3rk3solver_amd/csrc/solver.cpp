@@ -511,7 +511,9 @@ class SolverImpl final : public DeviceSolver {
     }
 
     void run_stage_kernels(int upto, double dt, int stage) override {
-        launch_reconstruct<R>(P_, L_.tile, lds_recon_, stream_, lanes_);
+        DevPtrs<R> P = P_;
+        P.storeFlat = 1;  // every limiter and face state can be fetched afterwards
+        launch_reconstruct<R>(P, L_.tile, lds_recon_, stream_, lanes_);
         if (upto > 0) launch_bvd<R>(P_, L_.tile, lds_bvd_, stream_);
         if (upto > 1) launch_flux<R>(P_, cfg_.R, cfg_.Cv, stream_);
         if (upto > 2) {
@@ -659,8 +661,11 @@ class SolverImpl final : public DeviceSolver {
         P_.gu = m_gu.as<v2>();
         P_.gv = m_gv.as<v2>();
         P_.gT = m_gT.as<v2>();
-        dalloc(m_lim, sizeof(v4) * nc);
-        P_.lim = m_lim.as<v4>();
+        {
+            std::vector<v4> lim(nc + 1);  // the last entry: a flat cell's limiters
+            lim[nc].x = lim[nc].y = lim[nc].z = lim[nc].w = (R)1;
+            P_.lim = put(m_lim, lim.data(), lim.size());
+        }
         dalloc(m_smooth, nc + nb);
         P_.smooth = m_smooth.as<int8_t>();
         dzero(P_.smooth, nc + nb);
@@ -670,6 +675,10 @@ class SolverImpl final : public DeviceSolver {
         dalloc(m_flat_prev, nc);
         P_.flat_prev = m_flat_prev.as<uint8_t>();
         dzero(P_.flat_prev, nc);
+        dalloc(m_fflat, 2 * nf);
+        P_.fflat = m_fflat.as<uint8_t>();
+        dzero(P_.fflat, 2 * nf);
+        P_.storeFlat = 0;
         dalloc(m_tlim, nc);
         P_.tlim = m_tlim.as<int8_t>();
         dzero(P_.tlim, nc);
@@ -836,7 +845,7 @@ class SolverImpl final : public DeviceSolver {
     DevMem m_W, m_U, m_Uold, m_vol, m_gp, m_gu, m_gv, m_gT, m_lim, m_smooth, m_ftype, m_scnt, m_ccnt, m_sten,
         m_slot_face, m_slot_d, m_slot_e, m_slot_dr, m_lsq, m_rbf, m_halo, m_more_ptr, m_halo_more, m_fcell, m_fgeo, m_fgeo32,
         m_fv, m_fvp, m_fvu, m_fvv, m_flux, m_flux32, m_bcell, m_blabel, m_bgeo, m_bval, m_dt, m_fvT, m_cinst, m_finst, m_tctl, m_res,
-        m_rbf_gp, m_fgd, m_fvg, m_flat_prev, m_tlim, m_tTVD, m_cen, m_fcen, m_fshift, m_fsf, m_fmag;
+        m_rbf_gp, m_fgd, m_fvg, m_flat_prev, m_fflat, m_tlim, m_tTVD, m_cen, m_fcen, m_fshift, m_fsf, m_fmag;
 };
 
 // A solver on relabelled cells and faces (compact_tile_order) that reads and
