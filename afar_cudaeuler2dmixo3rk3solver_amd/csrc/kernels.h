@@ -8,6 +8,7 @@
 namespace afar {
 
 constexpr int kCflBlocks = 1024;
+constexpr int kCflGroup = 32, kCflGroups = kCflBlocks / kCflGroup;  // blocks that share a ticket counter
 constexpr int kMaxSten = 20;  // largest stencil (the reference's limit, basicCUDAsolver.cpp:393-397)
 
 template <typename R> struct VT;
@@ -99,7 +100,7 @@ struct DevPtrs {
     const double4* bval;       // nb fixed values of label 6
     double* dt;                // device time step of each instance (ninst)
     double* dt_part;           // dt_cap partial minima of the CFL pass
-    unsigned int* dt_count;    // blocks of the CFL pass done
+    unsigned int* dt_count;    // tickets of the CFL pass: kCflGroups + 1 counters 128 bytes apart
     int dt_cap;                // capacity of dt_part: kCflBlocks or two per flux block, whichever is larger
     // Batches: ninst independent meshes stored one after the other (cells,
     // internal faces, boundary faces each contiguous per instance).  Each has
@@ -115,7 +116,9 @@ struct DevPtrs {
 };
 
 template <typename R> void launch_lsq(const DevPtrs<R>& p, hipStream_t s);
-template <typename R> void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, hipStream_t s);
+// host_dt (optional): pinned host memory that receives the time step too.
+template <typename R>
+void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, double* host_dt, hipStream_t s);
 // lanes: 1 = one thread per cell (any mesh); 4 = four threads per cell;
 // 2 = four threads per cell with the face work compacted (both: meshes whose
 // cells have at most four faces; 2 also tiles of at most 128 cells).

@@ -120,10 +120,12 @@ __device__ __forceinline__ double cfl_face_dt(const double4& g0, const double4& 
 
 // Each block reduces a contiguous chunk of faces (stride loop) to one
 // partial minimum; the last block to finish reduces the partials and stores
-// the time step on the device.  At most kCflBlocks partials, so only that
-// many same-address atomics per step.
+// the time step on the device and, for the host that waits for it, in pinned
+// host memory.  Blocks draw tickets by group of kCflGroup, the last of each
+// group one more: 1024 tickets on one address take 20 us (250k quads 31 us a
+// launch), on 32 addresses next to nothing (XX us).
 template <typename R>
-__global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double R_, double Cv, double CFL, int chunk) {
+__global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double R_, double Cv, double CFL, int chunk, double* host_dt) {
     const int blk = xcd_tile(blockIdx.x, gridDim.x);
     const int f0 = blk * chunk;
     const int f1 = min(p.nf, f0 + chunk);
@@ -138,13 +140,27 @@ __global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double R_, double Cv,
     const double m = block_min_256(dtf, wmin);
     if (threadIdx.x == 0) {
         __hip_atomic_store(&p.dt_part[blockIdx.x], m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __threadfence();
-        const unsigned t = atomicAdd(p.dt_count, 1u);
-        last = (t == gridDim.x - 1);
+        const unsigned g = blockIdx.x / kCflGroup, ngroups = (gridDim.x + kCflGroup - 1) / kCflGroup;
+        const unsigned size = min((unsigned)kCflGroup, gridDim.x - g * kCflGroup);
+        // counters one 128-byte line apart: the groups', then the launch's
+        unsigned* mine = p.dt_count + 32 * g;
+        unsigned* all = p.dt_count + 32 * kCflGroups;
+        last = 0;
+        // The partial is stored past the L2 (agent scope) and is waited for,
+        // and read past it below: no fence, which would write the L2 back.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (__hip_atomic_fetch_add(mine, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == size - 1) {
+            __hip_atomic_store(mine, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (ngroups == 1) {
+                last = 1;
+            } else if (__hip_atomic_fetch_add(all, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ngroups - 1) {
+                __hip_atomic_store(all, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                last = 1;
+            }
+        }
     }
     __syncthreads();
     if (!last) return;
-    __threadfence();
     double v = 1e5;
     for (int i = threadIdx.x; i < (int)gridDim.x; i += 256) {
         const double o = __hip_atomic_load(&p.dt_part[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -153,7 +169,7 @@ __global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double R_, double Cv,
     v = block_min_256(v, wmin);
     if (threadIdx.x == 0) {
         *p.dt = v;
-        atomicExch(p.dt_count, 0u);
+        if (host_dt) __hip_atomic_store(host_dt, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -1558,10 +1574,10 @@ void launch_lsq(const DevPtrs<R>& p, hipStream_t s) {
 static inline int pad8(int n) { return ((n + 7) / 8) * 8; }
 
 template <typename R>
-void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, hipStream_t s) {
+void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, double* host_dt, hipStream_t s) {
     const int nt = pad8(std::min(kCflBlocks, std::max(1, (p.nf + 255) / 256)));
     const int chunk = (p.nf + nt - 1) / nt;
-    hipLaunchKernelGGL(k_cfl<R>, dim3(nt), dim3(256), 0, s, p, Rg, Cv, CFL, chunk);
+    hipLaunchKernelGGL(k_cfl<R>, dim3(nt), dim3(256), 0, s, p, Rg, Cv, CFL, chunk, host_dt);
 }
 
 template <typename R, bool GP, int MS>
@@ -1678,7 +1694,7 @@ hipError_t set_lds_limits(size_t lds) {
 
 #define AFAR_INSTANTIATE(R)                                                                                        \
     template void launch_lsq<R>(const DevPtrs<R>&, hipStream_t);                                                  \
-    template void launch_cfl<R>(const DevPtrs<R>&, double, double, double, hipStream_t);                          \
+    template void launch_cfl<R>(const DevPtrs<R>&, double, double, double, double*, hipStream_t);                          \
     template void launch_reconstruct<R>(const DevPtrs<R>&, int, size_t, hipStream_t, int);                        \
     template void launch_bvd<R>(const DevPtrs<R>&, int, size_t, hipStream_t);                                     \
     template void launch_flux<R>(const DevPtrs<R>&, double, double, hipStream_t);                                 \

@@ -50,6 +50,25 @@ struct DevMem {
     template <typename T> T* as() const { return reinterpret_cast<T*>(p); }
 };
 
+// One double of pinned host memory, and its device address.
+struct PinnedDouble {
+    double *p = nullptr, *dev = nullptr;
+    ~PinnedDouble() {
+        if (p) (void)hipHostFree(p);
+    }
+    void alloc() {
+        check_hip(hipHostMalloc((void**)&p, sizeof(double), hipHostMallocMapped | hipHostMallocCoherent),
+                  "hipHostMalloc");
+        check_hip(hipHostGetDevicePointer((void**)&dev, p, 0), "hipHostGetDevicePointer");
+    }
+};
+
+inline void cpu_pause() {
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+}
+
 // The solver's stream: created here unless the caller gave one; destroyed
 // after the buffers (members declared after it) have enqueued their frees.
 struct StreamHolder {
@@ -126,6 +145,7 @@ class SolverImpl final : public DeviceSolver {
             sh_.own = true;
         }
         stream_ = sh_.s;
+        if (ninst() == 1) host_dt_.alloc();
         check_hip(hipEventCreate(&ev0_), "hipEventCreate");
         check_hip(hipEventCreate(&ev1_), "hipEventCreate");
         for (hipEvent_t& e : evq_) check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
@@ -166,12 +186,16 @@ class SolverImpl final : public DeviceSolver {
 
     double compute_dt() override {
         if (ninst() > 1) throw Error(1, "a batch steps with the device time step only");
-        launch_cfl<R>(P_, cfg_.R, cfg_.Cv, cfg_.CFL, stream_);
+        // The kernel's last block stores the value in pinned host memory, which
+        // the host polls: no copy, and no wait for the launch to retire.  The
+        // stored minimum is never NaN.
+        volatile double* dt = host_dt_.p;
+        *dt = std::nan("");
+        launch_cfl<R>(P_, cfg_.R, cfg_.Cv, cfg_.CFL, host_dt_.dev, stream_);
         check_hip(hipGetLastError(), "k_cfl");
-        double dt = 0.0;
-        check_hip(hipMemcpyAsync(&dt, P_.dt, sizeof(double), hipMemcpyDeviceToHost, stream_), "dt copy");
-        check_hip(hipStreamSynchronize(stream_), "dt sync");
-        return dt;
+        for (int i = 0; i < 200000 && *dt != *dt; ++i) cpu_pause();
+        if (*dt != *dt) check_hip(hipStreamSynchronize(stream_), "dt sync");  // earlier work still runs
+        return *dt;
     }
 
     void evolve(double dt) override {
@@ -412,7 +436,7 @@ class SolverImpl final : public DeviceSolver {
             check_hip(hipEventRecord(ev0_, stream_), "hipEventRecord");
             for (int r = 0; r < reps; ++r) {
                 switch (k) {
-                    case kKernCfl: launch_cfl<R>(P_, cfg_.R, cfg_.Cv, cfg_.CFL, stream_); break;
+                    case kKernCfl: launch_cfl<R>(P_, cfg_.R, cfg_.Cv, cfg_.CFL, nullptr, stream_); break;
                     case kKernRecon: launch_reconstruct<R>(P_, L_.tile, lds_recon_, stream_, lanes_); break;
                     case kKernBvd: launch_bvd<R>(P_, L_.tile, lds_bvd_, stream_); break;
                     case kKernFlux: launch_flux<R>(P_, cfg_.R, cfg_.Cv, stream_); break;
@@ -798,17 +822,17 @@ class SolverImpl final : public DeviceSolver {
         P_.res_part = m_res.as<double>();
         const int dt_cap = std::max(kCflBlocks, 2 * flux_blocks(L_.nf, L_.nb));
         const size_t dt_bytes = (sizeof(double) * ni + 255) / 256 * 256;
-        dalloc(m_dt, dt_bytes + 256 + sizeof(double) * dt_cap);
+        const size_t count_bytes = ((size_t)(kCflGroups + 1) * 128 + 255) / 256 * 256;
+        dalloc(m_dt, dt_bytes + count_bytes + sizeof(double) * dt_cap);
         P_.dt_cap = dt_cap;
         P_.dt = m_dt.as<double>();
         P_.dt_count = reinterpret_cast<unsigned int*>(m_dt.as<char>() + dt_bytes);
-        P_.dt_part = reinterpret_cast<double*>(m_dt.as<char>() + dt_bytes + 256);
+        P_.dt_part = reinterpret_cast<double*>(m_dt.as<char>() + dt_bytes + count_bytes);
+        dzero(P_.dt_count, count_bytes);
         {
             const std::vector<double> init_dt(ni, 1e5);
-            unsigned int zero = 0;
             check_hip(hipMemcpyAsync(P_.dt, init_dt.data(), sizeof(double) * ni, hipMemcpyHostToDevice, stream_),
                       "dt init");
-            check_hip(hipMemcpyAsync(P_.dt_count, &zero, 4, hipMemcpyHostToDevice, stream_), "dt init");
             synchronize();
         }
         upload_state();
@@ -828,6 +852,7 @@ class SolverImpl final : public DeviceSolver {
     BatchIndex bi_;
     DevLayout L_;
     DevPtrs<R> P_{};
+    PinnedDouble host_dt_;  // before the stream: freed after its last kernel
     StreamHolder sh_;  // before the buffers: destroyed after them
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
