@@ -85,7 +85,6 @@ struct afar_solver {
 struct afar_batch {
     std::unique_ptr<DeviceSolver> dev;
     BatchIndex idx;
-    std::vector<std::vector<int32_t>> perm;  // per instance: mesh cell -> caller cell
 };
 
 struct afar_device {
@@ -573,7 +572,7 @@ static int solver_create(const afar_mesh* h, const afar_schemes* s, const double
         sol->perm = h->m.perm;
         sol->nc = h->m.nc;
         sol->nb = h->m.nb;
-        sol->dev = make_device_solver(ra, cfg);
+        sol->dev = make_device_solver(ra, cfg, nullptr, sol->perm.data());
         *out = sol.release();
     });
 }
@@ -596,6 +595,7 @@ int afar_batch_create(int32_t n, const afar_mesh* const* meshes, const afar_sche
         need(out && meshes && W0 && s && n > 0, "bad arguments");
         auto b = std::make_unique<afar_batch>();
         RefArrays u;
+        std::vector<int32_t> out_pos;  // batch cell -> its instance's first cell + caller cell
         {
             std::vector<RefArrays> parts(n);
             std::vector<const RefArrays*> pp(n);
@@ -603,9 +603,10 @@ int afar_batch_create(int32_t n, const afar_mesh* const* meshes, const afar_sche
                 need(meshes[k] != nullptr && W0[k] != nullptr, "NULL mesh or state in the batch");
                 parts[k] = ref_arrays_of(meshes[k], s, W0[k]);
                 pp[k] = &parts[k];
-                b->perm.push_back(meshes[k]->m.perm);
             }
             u = union_ref_arrays(pp, b->idx);
+            for (int k = 0; k < n; ++k)
+                for (int32_t q : meshes[k]->m.perm) out_pos.push_back(b->idx.cell_off[k] + q);
         }
         SolverConfig cfg;
         cfg.R = s->R;
@@ -619,7 +620,7 @@ int afar_batch_create(int32_t n, const afar_mesh* const* meshes, const afar_sche
         cfg.reconLanes = s->reconLanes;
         need(s->cellOrder >= 0 && s->cellOrder <= 2, "cellOrder must be 0, 1 or 2");
         cfg.cellOrder = s->cellOrder;
-        b->dev = make_device_solver(u, cfg, &b->idx);
+        b->dev = make_device_solver(u, cfg, &b->idx, out_pos.data());
         *out = b.release();
     });
 }
@@ -685,11 +686,7 @@ int afar_batch_get_conserved(afar_batch* b, int32_t inst, double* U) {
     return guard([&] {
         need(b && U && inst >= 0 && inst < b->idx.ninst(), "bad arguments");
         const int c0 = b->idx.cell_off[inst], n = b->idx.cell_off[inst + 1] - c0;
-        std::vector<double> u(4 * (size_t)n);
-        b->dev->get_conserved_range(c0, n, u.data());
-        const auto& perm = b->perm[inst];
-        for (int i = 0; i < n; ++i)
-            for (int k = 0; k < 4; ++k) U[4 * (size_t)perm[i] + k] = u[4 * (size_t)i + k];
+        b->dev->read_conserved(c0, n, U);
     });
 }
 
@@ -697,15 +694,7 @@ int afar_batch_write_field(afar_batch* b, int32_t inst, double* W, int8_t* shock
     return guard([&] {
         need(b && inst >= 0 && inst < b->idx.ninst(), "bad arguments");
         const int c0 = b->idx.cell_off[inst], n = b->idx.cell_off[inst + 1] - c0;
-        std::vector<double> w(4 * (size_t)n);
-        std::vector<int8_t> t(n);
-        b->dev->get_primitive_range(c0, n, w.data(), t.data());
-        const auto& perm = b->perm[inst];
-        for (int i = 0; i < n; ++i) {
-            if (W)
-                for (int k = 0; k < 4; ++k) W[4 * (size_t)perm[i] + k] = w[4 * (size_t)i + k];
-            if (shock) shock[perm[i]] = t[i];
-        }
+        b->dev->read_fields(c0, n, W, shock, false);
     });
 }
 
@@ -803,27 +792,15 @@ int afar_solver_synchronize(afar_solver* h) {
 int afar_solver_write_field(afar_solver* h, double* W, double* ghost, int8_t* shock) {
     return guard([&] {
         need(h != nullptr, "NULL solver");
-        const int nc = h->nc, nb = h->nb;
-        std::vector<double> fd(4 * (size_t)(nc + nb));
-        std::vector<int8_t> sh(2 * (size_t)(nc + nb));
-        h->dev->copy_out(fd.data(), sh.data());
-        for (int i = 0; i < nc; ++i) {
-            const int o = h->perm[i];
-            if (W)
-                for (int k = 0; k < 4; ++k) W[4 * (size_t)o + k] = fd[4 * (size_t)i + k];
-            if (shock) shock[o] = sh[2 * (size_t)i + 1];
-        }
-        if (ghost) memcpy(ghost, fd.data() + 4 * (size_t)nc, sizeof(double) * 4 * nb);
+        if (W || shock) h->dev->read_fields(0, h->nc, W, shock, false);
+        if (ghost) h->dev->read_ghosts(ghost);
     });
 }
 
 int afar_solver_get_conserved(afar_solver* h, double* U) {
     return guard([&] {
         need(h && U, "NULL argument");
-        std::vector<double> u(4 * (size_t)h->nc);
-        h->dev->get_conserved(u.data());
-        for (int i = 0; i < h->nc; ++i)
-            for (int k = 0; k < 4; ++k) U[4 * (size_t)h->perm[i] + k] = u[4 * (size_t)i + k];
+        h->dev->read_conserved(0, h->nc, U);
     });
 }
 
@@ -1059,7 +1036,11 @@ int afar_copy_field_data_device_to_host(afar_field_pointer* host, afar_device* d
     return guard([&] {
         need(dev && dev->dev && host, "device not initialised");
         need(cellsNum == dev->ra.nc && totalBoundaryFacesNum == dev->ra.nb, "sizes differ from the upload");
-        dev->dev->copy_out(host->FD, host->shockIndicator);
+        const size_t nc = (size_t)cellsNum, nb = (size_t)totalBoundaryFacesNum;
+        if (host->FD || host->shockIndicator)
+            dev->dev->read_fields(0, (int)nc, host->FD, host->shockIndicator, true);
+        if (host->FD) dev->dev->read_ghosts(host->FD + 4 * nc);
+        if (host->shockIndicator) memset(host->shockIndicator + 2 * nc, 0, 2 * nb);  // pseudo-cells carry no flags
     });
 }
 

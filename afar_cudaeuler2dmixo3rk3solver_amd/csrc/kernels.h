@@ -139,6 +139,13 @@ template <typename R> void launch_residual_norm(const DevPtrs<R>& p, double* out
 template <typename R>
 void launch_update(const DevPtrs<R>& p, double Rg, double gamma, double dt, const double* dt_ptr, double b1, double b2,
                    double b3, int last, hipStream_t s);
+// Output in another cell order: rows idx[0..n) of the conserved state src, and
+// of the primitive state (as doubles) with the types or (pairs) the smoothness
+// flag and type of each.
+void launch_gather_state(const double4* src, const int32_t* idx, double4* dst, int n, hipStream_t s);
+template <typename R>
+void launch_gather_fields(const DevPtrs<R>& p, const int32_t* idx, double4* W, int8_t* flags, int pairs, int n,
+                          hipStream_t s);
 // Raises each reconstruction kernel's dynamic-LDS limit to lds minus its static LDS.
 template <typename R> hipError_t set_lds_limits(size_t lds);
 void launch_math_selftest(const double* x, double* out, int n, hipStream_t s);

@@ -233,51 +233,48 @@ class SolverImpl final : public DeviceSolver {
         return dt;
     }
 
-    void copy_out(double* FD, int8_t* shock) override {
-        const int nc = L_.nc, nb = L_.nb;
-        std::vector<v4> w(nc + nb);
-        std::vector<int8_t> s(nc + nb), t(nc);
-        check_hip(hipMemcpyAsync(w.data(), P_.W, sizeof(v4) * (nc + nb), hipMemcpyDeviceToHost, stream_), "W copy");
-        check_hip(hipMemcpyAsync(s.data(), P_.smooth, nc + nb, hipMemcpyDeviceToHost, stream_), "flag copy");
-        check_hip(hipMemcpyAsync(t.data(), P_.ftype, nc, hipMemcpyDeviceToHost, stream_), "type copy");
-        synchronize();
-        if (FD)
-            for (int i = 0; i < nc + nb; ++i) {
-                FD[4 * i] = w[i].x;
-                FD[4 * i + 1] = w[i].y;
-                FD[4 * i + 2] = w[i].z;
-                FD[4 * i + 3] = w[i].w;
-            }
-        if (shock)
-            for (int i = 0; i < nc + nb; ++i) {
-                shock[2 * i] = s[i];
-                shock[2 * i + 1] = i < nc ? t[i] : 0;
-            }
-    }
-
-    void get_conserved(double* U) override {
-        check_hip(hipMemcpyAsync(U, state_U(), sizeof(double4) * L_.nc, hipMemcpyDeviceToHost, stream_), "U copy");
+    void read_conserved(int o0, int n, double* U) override {
+        if (o0 < 0 || n < 0 || o0 + n > L_.nc) throw Error(1, "cell range out of bounds");
+        double4* st = staging();
+        launch_gather_state(state_U(), m_out_.as<const int32_t>() + o0, st, n, stream_);
+        check_hip(hipGetLastError(), "gather");
+        touch(U, sizeof(double4) * n);
+        check_hip(hipMemcpyAsync(U, st, sizeof(double4) * n, hipMemcpyDeviceToHost, stream_), "U copy");
         synchronize();
     }
 
-    void get_conserved_range(int c0, int n, double* U) override {
-        if (c0 < 0 || n < 0 || c0 + n > L_.nc) throw Error(1, "cell range out of bounds");
-        check_hip(hipMemcpyAsync(U, state_U() + c0, sizeof(double4) * n, hipMemcpyDeviceToHost, stream_), "U copy");
-        synchronize();
-    }
-
-    void get_primitive_range(int c0, int n, double* W, int8_t* type) override {
-        if (c0 < 0 || n < 0 || c0 + n > L_.nc) throw Error(1, "cell range out of bounds");
-        std::vector<v4> w(W ? n : 0);
-        if (W) check_hip(hipMemcpyAsync(w.data(), P_.W + c0, sizeof(v4) * n, hipMemcpyDeviceToHost, stream_), "W copy");
-        if (type) check_hip(hipMemcpyAsync(type, P_.ftype + c0, n, hipMemcpyDeviceToHost, stream_), "type copy");
-        synchronize();
-        for (int i = 0; i < (W ? n : 0); ++i) {
-            W[4 * (size_t)i] = w[i].x;
-            W[4 * (size_t)i + 1] = w[i].y;
-            W[4 * (size_t)i + 2] = w[i].z;
-            W[4 * (size_t)i + 3] = w[i].w;
+    void read_fields(int o0, int n, double* W, int8_t* flags, bool pairs) override {
+        if (o0 < 0 || n < 0 || o0 + n > L_.nc) throw Error(1, "cell range out of bounds");
+        double4* st = staging();
+        int8_t* fl = m_flags_.as<int8_t>();
+        launch_gather_fields<R>(P_, m_out_.as<const int32_t>() + o0, st, fl, pairs, n, stream_);
+        check_hip(hipGetLastError(), "gather");
+        if (W) {
+            touch(W, sizeof(double4) * n);
+            check_hip(hipMemcpyAsync(W, st, sizeof(double4) * n, hipMemcpyDeviceToHost, stream_), "W copy");
         }
+        if (flags) check_hip(hipMemcpyAsync(flags, fl, pairs ? 2 * n : n, hipMemcpyDeviceToHost, stream_), "flag copy");
+        synchronize();
+    }
+
+    void read_ghosts(double* g) override {
+        const int nb = L_.nb;
+        std::vector<v4> w(nb);
+        if (nb) check_hip(hipMemcpyAsync(w.data(), P_.W + L_.nc, sizeof(v4) * nb, hipMemcpyDeviceToHost, stream_), "W copy");
+        synchronize();
+        for (int b = 0; b < nb; ++b) {
+            g[4 * (size_t)b] = w[b].x;
+            g[4 * (size_t)b + 1] = w[b].y;
+            g[4 * (size_t)b + 2] = w[b].z;
+            g[4 * (size_t)b + 3] = w[b].w;
+        }
+    }
+
+    void set_output_order(const int32_t* out_pos) override {
+        std::vector<int32_t> idx(L_.nc);
+        for (int c = 0; c < L_.nc; ++c) idx[out_pos ? out_pos[c] : c] = c;
+        put(m_out_, idx.data(), idx.size());
+        dalloc(m_flags_, 2 * (size_t)L_.nc);
     }
 
     void reset_state() override { upload_state(); }
@@ -618,6 +615,23 @@ class SolverImpl final : public DeviceSolver {
         check_hip(hipGraphInstantiate(&graph_exec_, graph_, nullptr, nullptr, 0), "hipGraphInstantiate");
     }
 
+    // nc rows for the results on their way out: U, which the next step does not
+    // read while the state is in Uold, else a buffer of its own
+    double4* staging() {
+        if (state_in_uold_) return P_.U;
+        if (!m_stage_.p) {
+            std::lock_guard<std::mutex> lk(runtime_mutex());
+            dalloc(m_stage_, sizeof(double4) * L_.nc);
+        }
+        return m_stage_.as<double4>();
+    }
+    // Writes to every page of a result array before the copy that fills it, while
+    // the device is still stepping: the copy then meets no page fault.
+    static void touch(void* p, size_t bytes) {
+        volatile char* c = static_cast<char*>(p);
+        for (size_t i = 0; i < bytes; i += 4096) c[i] = 0;
+    }
+
     void dalloc(DevMem& m, size_t bytes) { m.alloc(bytes, stream_); }
     void dzero(void* p, size_t bytes) { check_hip(hipMemsetAsync(p, 0, bytes, stream_), "hipMemsetAsync"); }
     // n doubles uploaded in the kernels' precision: as they are in FP64,
@@ -867,6 +881,7 @@ class SolverImpl final : public DeviceSolver {
     double4* state_U() const { return state_in_uold_ ? P_.Uold : P_.U; }
     size_t lds_recon_ = 0, lds_bvd_ = 0, lds_m_off_ = 0, lds_bvd_sten_off_ = 0;
     int lanes_ = 1;  // threads per cell of the reconstruction kernel
+    DevMem m_out_, m_flags_, m_stage_;  // output order (cell at each position), flags and states on their way out
     DevMem m_W, m_U, m_Uold, m_vol, m_gp, m_gu, m_gv, m_gT, m_lim, m_smooth, m_ftype, m_scnt, m_ccnt, m_sten,
         m_slot_face, m_slot_d, m_slot_e, m_slot_dr, m_lsq, m_rbf, m_halo, m_more_ptr, m_halo_more, m_fcell, m_fgeo, m_fgeo32,
         m_fv, m_fvp, m_fvu, m_fvv, m_flux, m_flux32, m_bcell, m_blabel, m_bgeo, m_bval, m_dt, m_fvT, m_cinst, m_finst, m_tctl, m_res,
@@ -886,25 +901,15 @@ class RelabeledSolver final : public DeviceSolver {
     void evolve_auto(int nsteps) override { in_->evolve_auto(nsteps); }
     void synchronize() override { in_->synchronize(); }
     bool idle() override { return in_->idle(); }
-    void copy_out(double* FD, int8_t* shock) override {
-        std::vector<double> f(FD ? 4 * (size_t)(nc_ + nb_) : 0);
-        std::vector<int8_t> s(shock ? 2 * (size_t)(nc_ + nb_) : 0);
-        in_->copy_out(FD ? f.data() : nullptr, shock ? s.data() : nullptr);
-        for (int i = 0; i < nc_ + nb_; ++i) {
-            const size_t j = i < nc_ ? (size_t)r_.cell_new[i] : (size_t)i;
-            if (FD)
-                for (int k = 0; k < 4; ++k) FD[4 * (size_t)i + k] = f[4 * j + k];
-            if (shock) {
-                shock[2 * (size_t)i] = s[2 * j];
-                shock[2 * (size_t)i + 1] = s[2 * j + 1];
-            }
-        }
+    void read_conserved(int o0, int n, double* U) override { in_->read_conserved(o0, n, U); }
+    void read_fields(int o0, int n, double* W, int8_t* flags, bool pairs) override {
+        in_->read_fields(o0, n, W, flags, pairs);
     }
-    void get_conserved(double* U) override {
-        std::vector<double> u(4 * (size_t)nc_);
-        in_->get_conserved(u.data());
-        for (int i = 0; i < nc_; ++i)
-            for (int k = 0; k < 4; ++k) U[4 * (size_t)i + k] = u[4 * (size_t)r_.cell_new[i] + k];
+    void read_ghosts(double* g) override { in_->read_ghosts(g); }
+    void set_output_order(const int32_t* out_pos) override {
+        std::vector<int32_t> p(nc_);
+        for (int j = 0; j < nc_; ++j) p[j] = out_pos ? out_pos[r_.cell_old[j]] : r_.cell_old[j];
+        in_->set_output_order(p.data());
     }
     void set_conserved(const double* U) override {
         std::vector<double> u(4 * (size_t)nc_);
@@ -915,27 +920,6 @@ class RelabeledSolver final : public DeviceSolver {
     double last_dt() override { return in_->last_dt(); }
     int ninst() const override { return in_->ninst(); }
     void last_dts(double* out) override { in_->last_dts(out); }
-    void get_conserved_range(int c0, int n, double* U) override {
-        int lo, hi;
-        span(c0, n, lo, hi);
-        std::vector<double> u(4 * (size_t)(hi - lo));
-        if (hi > lo) in_->get_conserved_range(lo, hi - lo, u.data());
-        for (int i = 0; i < n; ++i)
-            for (int k = 0; k < 4; ++k) U[4 * (size_t)i + k] = u[4 * (size_t)(r_.cell_new[c0 + i] - lo) + k];
-    }
-    void get_primitive_range(int c0, int n, double* W, int8_t* type) override {
-        int lo, hi;
-        span(c0, n, lo, hi);
-        std::vector<double> w(W ? 4 * (size_t)(hi - lo) : 0);
-        std::vector<int8_t> t(type ? (size_t)(hi - lo) : 0);
-        if (hi > lo) in_->get_primitive_range(lo, hi - lo, W ? w.data() : nullptr, type ? t.data() : nullptr);
-        for (int i = 0; i < n; ++i) {
-            const size_t j = (size_t)(r_.cell_new[c0 + i] - lo);
-            if (W)
-                for (int k = 0; k < 4; ++k) W[4 * (size_t)i + k] = w[4 * j + k];
-            if (type) type[i] = t[j];
-        }
-    }
     void reset_state() override { in_->reset_state(); }
     void set_time(int inst, double t, double t_end) override { in_->set_time(inst, t, t_end); }
     void get_time(double* t, double* steps) override { in_->get_time(t, steps); }
@@ -992,17 +976,6 @@ class RelabeledSolver final : public DeviceSolver {
     }
 
    private:
-    // the device range holding mesh cells [c0, c0+n)
-    void span(int c0, int n, int& lo, int& hi) const {
-        if (c0 < 0 || n < 0 || c0 + n > nc_) throw Error(1, "cell range out of bounds");
-        lo = nc_;
-        hi = 0;
-        for (int i = c0; i < c0 + n; ++i) {
-            lo = std::min(lo, r_.cell_new[i]);
-            hi = std::max(hi, r_.cell_new[i] + 1);
-        }
-        if (hi < lo) lo = hi = 0;
-    }
     std::unique_ptr<DeviceSolver> in_;
     Relabel r_;
     int nc_, nf_, nb_;
@@ -1017,7 +990,7 @@ std::unique_ptr<DeviceSolver> make_impl(RefArrays&& ra, DevLayout&& L, const Sol
 }  // namespace
 
 std::unique_ptr<DeviceSolver> make_device_solver(const RefArrays& ra, const SolverConfig& cfg,
-                                                 const BatchIndex* bi) {
+                                                 const BatchIndex* bi, const int32_t* out_pos) {
     if (ra.nc <= 0) throw Error(1, "empty mesh");
     // host-side work (copies, relabelling, the device layout) runs before the
     // library's lock is taken, so that solvers prepared on several threads
@@ -1026,7 +999,9 @@ std::unique_ptr<DeviceSolver> make_device_solver(const RefArrays& ra, const Solv
         RefArrays copy = ra;
         DevLayout L = solver_layout(copy, cfg);
         std::lock_guard<std::mutex> lk(runtime_mutex());
-        return make_impl(std::move(copy), std::move(L), cfg, bi);
+        auto s = make_impl(std::move(copy), std::move(L), cfg, bi);
+        s->set_output_order(out_pos);
+        return s;
     }
     BatchIndex one;
     if (!bi) {
@@ -1044,8 +1019,10 @@ std::unique_ptr<DeviceSolver> make_device_solver(const RefArrays& ra, const Solv
         DevLayout L = solver_layout(rl, cfg);
         std::lock_guard<std::mutex> lk(runtime_mutex());
         in = make_impl(std::move(rl), std::move(L), cfg, bi);
+        in = std::unique_ptr<DeviceSolver>(new RelabeledSolver(std::move(in), std::move(r), ra.nc, ra.nf, ra.nb));
+        in->set_output_order(out_pos);
     }
-    return std::unique_ptr<DeviceSolver>(new RelabeledSolver(std::move(in), std::move(r), ra.nc, ra.nf, ra.nb));
+    return in;
 }
 
 }  // namespace afar

@@ -59,17 +59,20 @@ class DeviceSolver {
     virtual void evolve_auto(int nsteps) = 0;           // CFL + step on the device, graph replay
     virtual void synchronize() = 0;
     virtual bool idle() = 0;  // all enqueued work done (does not wait)
-    virtual void copy_out(double* FD, int8_t* shock) = 0;  // FD 4*(nc+nb); shock 2*(nc+nb) interleaved
-    virtual void get_conserved(double* U) = 0;          // 4*nc
     virtual void set_conserved(const double* U) = 0;    // also recomputes W and ghosts
     virtual double last_dt() = 0;
     // Instances of a batch (1 for one mesh) and the time step of each.
     virtual int ninst() const = 0;
     virtual void last_dts(double* out) = 0;
-    // Cells [c0, c0+n): conserved state (4n); primitive state (4n) and final
-    // reconstruction types (n); either output may be NULL.
-    virtual void get_conserved_range(int c0, int n, double* U) = 0;
-    virtual void get_primitive_range(int c0, int n, double* W, int8_t* type) = 0;
+    // Results in the caller's order (make_device_solver's out_pos), gathered on
+    // the device: of positions [o0, o0 + n) the conserved state (4n), and the
+    // primitive state (4n) with the final reconstruction types (n) or, with
+    // pairs, (smoothness flag, type) each (2n); either output may be NULL.
+    // read_ghosts: the boundary pseudo-cells' states (4*nb).
+    virtual void read_conserved(int o0, int n, double* U) = 0;
+    virtual void read_fields(int o0, int n, double* W, int8_t* flags, bool pairs) = 0;
+    virtual void read_ghosts(double* g) = 0;
+    virtual void set_output_order(const int32_t* out_pos) = 0;
     // Back to the state the solver was created with (or last given to
     // set_conserved); the device clock is not changed.
     virtual void reset_state() = 0;
@@ -101,8 +104,9 @@ class DeviceSolver {
 
 // bi: instance offsets when ra is a batch (union_ref_arrays), else nullptr.
 // A batch steps with the device time step only (evolve_auto, time_steps).
+// out_pos: position of each of ra's cells in the results (nullptr: ra's order).
 std::unique_ptr<DeviceSolver> make_device_solver(const RefArrays& ra, const SolverConfig& cfg,
-                                                 const BatchIndex* bi = nullptr);
+                                                 const BatchIndex* bi = nullptr, const int32_t* out_pos = nullptr);
 void check_hip(hipError_t e, const char* what);
 
 }  // namespace afar
