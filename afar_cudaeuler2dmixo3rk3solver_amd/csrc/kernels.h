@@ -65,7 +65,8 @@ struct DevPtrs {
     const double* fmag;        // nf magSf
     R* slot_dr;                // sliced ELL, |slot_e| in the kernels' precision (written by K3)
     typename VT<R>::v2* lsq;   // sliced ELL, least-squares weights
-    const R* rbf;              // sliced ELL, RBF coefficients (face slot, stencil member)
+    int rbfRow;                // elements of a row of coefficients
+    const R* rbf;              // RBF coefficients: maxC rows per slice (DevLayout::rbf_at)
     int hfix, hcap;            // halo ids per row, capacity of the LDS halo (the dummy member follows it)
     const int32_t* halo;       // ntiles rows of hfix ids
     const int32_t* more_ptr;   // ntiles+1, ids of the longer lists past their row
@@ -87,7 +88,7 @@ struct DevPtrs {
     // extension (faceQuadrature): flux at ngp points per internal face
     int ngp;                   // 0: face centre only (reference)
     double gpw[4];             // point weights, sum 1
-    const R* rbf_gp;           // sliced ELL, RBF coefficients (point, face slot, stencil member)
+    const R* rbf_gp;           // RBF coefficients at the points: ngp * maxC rows per slice
     const typename VT<R>::v4* fgd;  // ngp*nf: point - owner centre (x, y), point - neighbour centre (z, w),
                                     // in the kernels' precision
     typename VT<R>::v4* fvg;   // ngp*2*nf reconstructed states at the points, [(g*nf + f)*2 + side]

@@ -203,6 +203,14 @@ __device__ __forceinline__ void store_face_state(const DevPtrs<R>& p, int i, con
     p.fvT[i] = o.w;
 }
 
+// Coefficient i of cell c in row k of K rows per slice (DevLayout::rbf_at).
+template <typename R>
+__device__ __forceinline__ R rbf_at(const R* rbf, int rbfRow, int c, int k, int K, int i) {
+    constexpr int V = 16 / sizeof(R);
+    const R* row = rbf + ((size_t)(c >> 6) * K + k) * rbfRow;
+    return i == 0 ? row[c & 63] : row[64 + ((i - 1) / V * 64 + (c & 63)) * V + (i - 1) % V];
+}
+
 template <typename R>
 __device__ __forceinline__ void limiter_process(R& lim, R& phif, R phic, R phiMax, R phiMin, R gx, R gy, R dx, R dy) {
     // cudaLimiter.h:35-50
@@ -256,7 +264,7 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
     if (c >= p.nc) return;
     const uint16_t* sSt = sRows + tid * p.stenW;  // this cell's members
     const int S = p.scnt[c], C = p.ccnt[c];
-    const int maxS = p.maxS, maxC = p.maxC, KR = maxC * (maxS + 1);
+    const int maxC = p.maxC;
     const v4 wc = sW[tid];
 
     R gpx = 0, gpy = 0, guxx = 0, guyx = 0, guxy = 0, guyy = 0, gTx = 0, gTy = 0;
@@ -366,12 +374,12 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
         const R fraction = sqrt(dx * dx + dy * dy) / deltaR;
         const int nbl = sSt[fi];
 
-        const R* a = p.rbf + sell(c, fi * (maxS + 1), KR);  // row stride 64
-        R coef = a[0];
+        auto at = [&](int m) { return rbf_at(p.rbf, p.rbfRow, c, fi, maxC, m); };
+        R coef = at(0);
         R pf = coef * wc.x, uxf = coef * wc.y, uyf = coef * wc.z, Tf = coef * wc.w;
         for (int ci = 0; ci < S; ++ci) {
             const v4 wj = sW[sSt[ci]];
-            coef = a[(size_t)(ci + 1) * 64];
+            coef = at(ci + 1);
             pf += coef * wj.x;
             uxf += coef * wj.y;
             uyf += coef * wj.z;
@@ -394,12 +402,12 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
         store_face_state(p, 2 * f + isNei, o);
         if constexpr (GP)
         for (int g = 0; g < p.ngp; ++g) {  // flux points (extension), as in k_reconstruct_q
-            const R* ag = p.rbf_gp + sell(c, (g * maxC + fi) * (maxS + 1), p.ngp * KR);
-            R cg = ag[0];
+            auto atg = [&](int m) { return rbf_at(p.rbf_gp, p.rbfRow, c, g * maxC + fi, p.ngp * maxC, m); };
+            R cg = atg(0);
             R pg = cg * wc.x, uxg = cg * wc.y, uyg = cg * wc.z, Tg = cg * wc.w;
             for (int ci = 0; ci < S; ++ci) {
                 const v4 wj = sW[sSt[ci]];
-                cg = ag[(size_t)(ci + 1) * 64];
+                cg = atg(ci + 1);
                 pg += cg * wj.x;
                 uxg += cg * wj.y;
                 uyg += cg * wj.z;
@@ -454,6 +462,24 @@ template <int X, typename T> __device__ __forceinline__ T quad_xor(T x) {
     return dpp_move<X == 1 ? 0xB1 : 0x4E>(x);  // quad_perm [1,0,3,2] and [2,3,0,1]
 }
 
+// A 16-byte group of coefficients.  Rows of single members (4 or 8 bytes a lane
+// and load, up to 17 loads) kept the reconstruction waiting on the loads
+// themselves: 740k mixed 79.3 -> 74.6 us with groups, 1.5M FP64 189 -> 184.5,
+// 20k quads 8.4 -> 7.7, 17k 8.3 -> 7.5.
+template <typename R> struct CoefGroup;
+template <> struct CoefGroup<double> {
+    using type = double2;
+    static __device__ __forceinline__ type splat(double x) { return type{x, x}; }
+    static __device__ __forceinline__ double get(const type& g, int i) { return i ? g.y : g.x; }
+};
+template <> struct CoefGroup<float> {
+    using type = float4;
+    static __device__ __forceinline__ type splat(float x) { return type{x, x, x, x}; }
+    static __device__ __forceinline__ float get(const type& g, int i) {
+        return i == 0 ? g.x : i == 1 ? g.y : i == 2 ? g.z : g.w;
+    }
+};
+
 // The largest of the values below 32 that x has in the lanes where m holds (0
 // if there is none): the same in every lane.
 __device__ __forceinline__ int wave_max32(int x, bool m) {
@@ -493,12 +519,12 @@ __device__ __forceinline__ int wave_max32(int x, bool m) {
 #ifndef AFAR_RECONQ_WPE_F
 #define AFAR_RECONQ_WPE_F 7
 #endif
-// The float flux-quadrature instantiation holds more values and asks for one
-// wave fewer, so that it does not spill.
-template <typename R, bool GP> struct ReconQWaves {
-    static constexpr int value = sizeof(R) == 8 ? AFAR_RECONQ_WPE_D : AFAR_RECONQ_WPE_F - (GP ? 1 : 0);
+// The float instantiations for flux quadrature and for stencils of 20 hold more
+// values and ask for one wave fewer, so that they do not spill.
+template <typename R, bool GP, int MS> struct ReconQWaves {
+    static constexpr int value = sizeof(R) == 8 ? AFAR_RECONQ_WPE_D : AFAR_RECONQ_WPE_F - (GP || MS > 16 ? 1 : 0);
 };
-#define AFAR_RECONQ_ATTR __attribute__((amdgpu_waves_per_eu(ReconQWaves<R, GP>::value, 8)))
+#define AFAR_RECONQ_ATTR __attribute__((amdgpu_waves_per_eu(ReconQWaves<R, GP, MS>::value, 8)))
 
 template <typename R, int TILE, bool GP, int MS>
 __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(DevPtrs<R> p) {
@@ -522,7 +548,7 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     const int t = threadIdx.x;
     const int lc = t >> 2, k = t & 3;
     const int c0 = tile * TILE, c = c0 + lc;
-    const int maxC = p.maxC, KR = maxC * (p.maxS + 1), nf = p.nf, SW = p.stenW;
+    const int maxC = p.maxC, nf = p.nf, SW = p.stenW;
     // Cell and slot arrays are addressed from bases the wavefront shares (its
     // 16 cells lie in one slice) with small lane offsets: scalar address
     // arithmetic instead of 64-bit vector arithmetic (with tTVD stored in slot
@@ -581,19 +607,23 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     // round already (flat_prev only schedules loads; results do not depend on
     // it).  The row count is the wavefront's: a cell of a shorter stencil reads
     // its padding (-0.0), which shares the other cells' 128-byte segments.
-    R cf[MS + 1];
+    constexpr int V = 16 / sizeof(R), NG = (MS + V - 1) / V;  // members per 16-byte group, groups
+    using G = typename CoefGroup<R>::type;
+    R cf0 = (R)-0.0;  // the cell's own coefficient
+    G cf[NG];         // the members'
     R deltaR = 0;
-    const R* a = p.rbf + slice * KR * 64;
-    const unsigned a0 = k * (p.maxS + 1) * 64 + cl;  // row stride 64
+    const R* a = p.rbf + slice * maxC * p.rbfRow;  // this slice's rows; lane k's at k * rbfRow
+    const unsigned a0 = k * p.rbfRow + cl, a1 = (k * p.rbfRow + 64) / V + cl;
 #pragma unroll
-    for (int i = 0; i <= MS; ++i) cf[i] = (R)-0.0;
+    for (int i = 0; i < NG; ++i) cf[i] = CoefGroup<R>::splat((R)-0.0);
     auto load_coefficients = [&](bool need) {
         const int rows = wave_max32(S, need);
         if (need) {
             if constexpr (!GEO) deltaR = slots(p.slot_dr)[row_k];
+            cf0 = a[a0];
 #pragma unroll
-            for (int i = 0; i <= MS; ++i)
-                if (i <= rows) cf[i] = (a + i * 64)[a0];
+            for (int i = 0; i < NG; ++i)
+                if (i * V < rows) cf[i] = (reinterpret_cast<const G*>(a) + i * 64)[a1];
         }
     };
     const bool early = live && !wasFlat;
@@ -761,26 +791,31 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
         return;
     }
 
-    // RBF sums, members four at a time up to the wavefront's longest stencil:
-    // the states of a round are requested together, and a cell that has no
-    // further members adds -0.0 * 1.
-    R pf = cf[0] * wc.x, uxf = cf[0] * wc.y, uyf = cf[0] * wc.z, Tf = cf[0] * wc.w;
+    // RBF sums, a group of members at a time up to the wavefront's longest
+    // stencil: the states of a group are requested together, and a cell that
+    // has no further members adds -0.0 * 1.
+    R pf = cf0 * wc.x, uxf = cf0 * wc.y, uyf = cf0 * wc.z, Tf = cf0 * wc.w;
     {
         const int rows = wave_max32(S, live);
         uint4 ids = row0;
 #pragma unroll
-        for (int j = 0; j < MS; j += 2) {
+        for (int j = 0; j < NG * V; j += V) {
             if (j < rows) {
                 if (j == 8 || j == 16) ids = row[j / 8];
-                const unsigned w2 = (j & 4) ? ((j & 2) ? ids.w : ids.z) : ((j & 2) ? ids.y : ids.x);
-                const v4 w4[2] = {sW[w2 & 0xffffu], sW[w2 >> 16]};
+                const unsigned w[4] = {ids.x, ids.y, ids.z, ids.w};
+                v4 m[V];
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const R coef = cf[j + i + 1];
-                    pf += coef * w4[i].x;
-                    uxf += coef * w4[i].y;
-                    uyf += coef * w4[i].z;
-                    Tf += coef * w4[i].w;
+                for (int i = 0; i < V; ++i) {
+                    const int h = (j + i) & 7;
+                    m[i] = sW[(h & 1) ? w[h >> 1] >> 16 : w[h >> 1] & 0xffffu];
+                }
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const R coef = CoefGroup<R>::get(cf[j / V], i);
+                    pf += coef * m[i].x;
+                    uxf += coef * m[i].y;
+                    uyf += coef * m[i].z;
+                    Tf += coef * m[i].w;
                 }
             }
         }
@@ -816,12 +851,12 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
         // or the unlimited linear state where the compact range is flat
         if constexpr (GP)
         for (int g = 0; g < p.ngp; ++g) {
-            const R* ag = p.rbf_gp + sell(c, (g * maxC + k) * (p.maxS + 1), p.ngp * KR);
-            R cg = ag[0];
+            auto atg = [&](int m) { return rbf_at(p.rbf_gp, p.rbfRow, c, g * maxC + k, p.ngp * maxC, m); };
+            R cg = atg(0);
             R pg = cg * wc.x, uxg = cg * wc.y, uyg = cg * wc.z, Tg = cg * wc.w;
             for (int ci = 0; ci < S; ++ci) {
                 const v4 wj = sW[sRows[lc * SW + ci]];
-                cg = ag[(size_t)(ci + 1) * 64];
+                cg = atg(ci + 1);
                 pg += cg * wj.x;
                 uxg += cg * wj.y;
                 uyg += cg * wj.z;

@@ -456,7 +456,7 @@ void global_stencil_from_blocks(int nc, int maxS, int maxLB, const uint8_t* S, c
     }
 }
 
-DevLayout make_dev_layout(const RefArrays& ra, int tile) {
+DevLayout make_dev_layout(const RefArrays& ra, int tile, int precision) {
     if (tile != 64 && tile != 128 && tile != 256) throw Error(1, "tile must be 64, 128 or 256");
     DevLayout L;
     const int nc = ra.nc, nf = ra.nf, nb = ra.nb, maxS = ra.maxS, maxC = ra.maxC;
@@ -469,7 +469,6 @@ DevLayout make_dev_layout(const RefArrays& ra, int tile) {
     L.nwaves = (nc + 63) / 64;
     L.ntiles = (nc + tile - 1) / tile;
     const size_t nslot = (size_t)L.nwaves * maxC * 64;
-    const int KR = maxC * (maxS + 1);
     L.scnt = ra.stencilSize;
     L.ccnt = ra.compactStencilSize;
     L.stenW = std::max(8, (maxS + 7) & ~7);
@@ -477,14 +476,16 @@ DevLayout make_dev_layout(const RefArrays& ra, int tile) {
     L.slot_face.assign(nslot, 0);
     L.slot_d.assign(2 * nslot, 0.0);
     L.slot_e.assign(2 * nslot, 0.0);
-    // Rows past a cell's stencil hold -0.0 and their ids name a dummy member of
+    // Coefficients past a cell's stencil are -0.0 and their ids name a dummy member of
     // state 1: the terms -0.0 * 1 that a whole wavefront's loop adds for a cell
     // of a shorter stencil leave every sum as it is.
-    L.rbf.assign((size_t)L.nwaves * KR * 64, -0.0);
+    L.rbfV = precision == 1 ? 4 : 2;
+    L.rbfRow = 64 * (1 + (maxS + L.rbfV - 1) / L.rbfV * L.rbfV);
+    L.rbf.assign((size_t)L.nwaves * maxC * L.rbfRow, -0.0);
     L.ngp = ra.ngp;
     L.gpw = ra.GPW;
     L.fgd = ra.GPD;
-    L.rbf_gp.assign((size_t)L.nwaves * ra.ngp * KR * 64, -0.0);
+    L.rbf_gp.assign((size_t)L.nwaves * ra.ngp * maxC * L.rbfRow, -0.0);
     L.vol = ra.cellVolume;
     const double* CELL = ra.CELL.data();
     const double* FACE = ra.FACE.data();
@@ -576,12 +577,12 @@ DevLayout make_dev_layout(const RefArrays& ra, int tile) {
                     }
                     const int side = sf < 0;
                     const double* a = &ra.RBFbasis[(size_t)2 * (maxS + 1) * f + (size_t)side * (maxS + 1)];
-                    for (int i = 0; i <= ra.stencilSize[c]; ++i) L.rbf[L.sell(c, fi * (maxS + 1) + i, KR)] = a[i];
+                    for (int i = 0; i <= ra.stencilSize[c]; ++i) L.rbf[L.rbf_at(c, fi, maxC, i)] = a[i];
                     for (int g = 0; g < ra.ngp; ++g) {
                         const double* ag =
                             &ra.RBFgp[(((size_t)g * nf + f) * 2 + side) * (size_t)(maxS + 1)];
                         for (int i = 0; i <= ra.stencilSize[c]; ++i)
-                            L.rbf_gp[L.sell(c, (g * maxC + fi) * (maxS + 1) + i, ra.ngp * KR)] = ag[i];
+                            L.rbf_gp[L.rbf_at(c, g * maxC + fi, ra.ngp * maxC, i)] = ag[i];
                     }
                 } else {
                     const int b = f - nf;

@@ -65,7 +65,12 @@ struct DevLayout {
     std::vector<int32_t> slot_face;       // nwaves*maxC*64, +-(f+1), 0 = padding
     std::vector<double> slot_d;           // 2 per slot: face centre - cell centre
     std::vector<double> slot_e;           // 2 per slot: compact neighbour - cell centre
-    std::vector<double> rbf;              // nwaves*maxC*(maxS+1)*64, padding -0.0
+    // RBF coefficients of a slot (rbf_row(): rbfRow elements): the cell's own
+    // for the 64 cells of a slice, then the members' in groups of rbfV (16
+    // bytes in the kernels' precision), a group of each cell side by side.
+    // Padding is -0.0.
+    int rbfV = 2, rbfRow = 0;
+    std::vector<double> rbf;              // nwaves*maxC rows
     // Global ids of a tile's halo members: the first hfix in a row of fixed
     // width (a short list repeats the tile's first cell), the rest of the few
     // longer lists in halo_more[more_ptr[tile] .. more_ptr[tile + 1]).  hcap:
@@ -84,12 +89,19 @@ struct DevLayout {
     // extension (faceQuadrature): flux points
     int ngp = 0;
     std::vector<double> gpw;              // ngp
-    std::vector<double> rbf_gp;           // per slot and point: element (g*maxC + k)*(maxS+1) + i, width 64
+    std::vector<double> rbf_gp;           // nwaves*ngp*maxC rows: row g*maxC + k
     std::vector<double> fgd;              // 4*ngp*nf as RefArrays::GPD
     size_t sell(int c, int k, int K) const { return ((size_t)(c >> 6) * K + k) * 64 + (c & 63); }
+    // coefficient i (0: the cell's own) of cell c in row k of K per slice
+    size_t rbf_at(int c, int k, int K, int i) const {
+        const size_t row = ((size_t)(c >> 6) * K + k) * rbfRow;
+        if (i == 0) return row + (c & 63);
+        return row + 64 + ((size_t)((i - 1) / rbfV) * 64 + (c & 63)) * rbfV + (i - 1) % rbfV;
+    }
 };
 
-DevLayout make_dev_layout(const RefArrays& ra, int tile);
+// precision: 0 FP64, 1 FP32-mixed (the grouping of the RBF coefficients).
+DevLayout make_dev_layout(const RefArrays& ra, int tile, int precision = 0);
 
 // A batch of independent meshes as one: the instances' cells, internal
 // faces, boundary faces (pseudo-cells) and patches each follow one another,

@@ -110,10 +110,10 @@ size_t lds_limit() {
 // 16-byte rows of ids take up to 14 bytes a cell and 48 more than the bare
 // states and ids: a tile that only they push over the LDS limit is halved.
 DevLayout solver_layout(const RefArrays& ra, const SolverConfig& cfg) {
-    DevLayout L = make_dev_layout(ra, cfg.tile);
+    DevLayout L = make_dev_layout(ra, cfg.tile, cfg.precision);
     const size_t cap = lds_limit();
     if (cfg.tile > 64 && recon_lds(L, cfg, L.hcap + 1, L.stenW) > cap && recon_lds(L, cfg, L.maxHalo, L.maxS) <= cap)
-        L = make_dev_layout(ra, cfg.tile / 2);
+        L = make_dev_layout(ra, cfg.tile / 2, cfg.precision);
     return L;
 }
 
@@ -123,7 +123,7 @@ class SolverImpl final : public DeviceSolver {
     using v2 = typename VT<R>::v2;
 
    public:
-    // ra and its device layout L (make_dev_layout(ra, cfg.tile)) are built by
+    // ra and its device layout L (make_dev_layout(ra, cfg.tile, cfg.precision)) are built by
     // the caller, outside the library's lock, and moved in.
     SolverImpl(RefArrays&& ra, DevLayout&& L, const SolverConfig& cfg, const BatchIndex* bi)
         : ra_(std::move(ra)), L_(std::move(L)) {
@@ -732,6 +732,7 @@ class SolverImpl final : public DeviceSolver {
         dzero(P_.slot_dr, sizeof(R) * nslot);
         dalloc(m_lsq, sizeof(v2) * nslot);
         P_.lsq = m_lsq.as<v2>();
+        P_.rbfRow = L_.rbfRow;
         P_.rbf = put_as_R(m_rbf, L_.rbf.data(), L_.rbf.size());
         P_.halo = put(m_halo, L_.halo.data(), L_.halo.size());
         P_.more_ptr = put(m_more_ptr, L_.more_ptr.data(), L_.more_ptr.size());
