@@ -519,10 +519,11 @@ __device__ __forceinline__ int wave_max32(int x, bool m) {
 #ifndef AFAR_RECONQ_WPE_F
 #define AFAR_RECONQ_WPE_F 7
 #endif
-// The float instantiations for flux quadrature and for stencils of 20 hold more
-// values and ask for one wave fewer, so that they do not spill.
+// The instantiations for flux quadrature and (float) for stencils of 20 hold
+// more values and ask for fewer waves, so that they do not spill.
 template <typename R, bool GP, int MS> struct ReconQWaves {
-    static constexpr int value = sizeof(R) == 8 ? AFAR_RECONQ_WPE_D : AFAR_RECONQ_WPE_F - (GP || MS > 16 ? 1 : 0);
+    static constexpr int value = sizeof(R) == 8 ? AFAR_RECONQ_WPE_D - (GP ? 1 : 0)
+                                                : AFAR_RECONQ_WPE_F - (GP ? 2 : MS > 16 ? 1 : 0);
 };
 #define AFAR_RECONQ_ATTR __attribute__((amdgpu_waves_per_eu(ReconQWaves<R, GP, MS>::value, 8)))
 
@@ -794,9 +795,9 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     // RBF sums, a group of members at a time up to the wavefront's longest
     // stencil: the states of a group are requested together, and a cell that
     // has no further members adds -0.0 * 1.
-    R pf = cf0 * wc.x, uxf = cf0 * wc.y, uyf = cf0 * wc.z, Tf = cf0 * wc.w;
-    {
-        const int rows = wave_max32(S, live);
+    const int rows = wave_max32(S, live);
+    auto rbf_sum = [&](R own, const G(&g)[NG], v4& o) {
+        o = v4{own * wc.x, own * wc.y, own * wc.z, own * wc.w};
         uint4 ids = row0;
 #pragma unroll
         for (int j = 0; j < NG * V; j += V) {
@@ -811,15 +812,18 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
                 }
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const R coef = CoefGroup<R>::get(cf[j / V], i);
-                    pf += coef * m[i].x;
-                    uxf += coef * m[i].y;
-                    uyf += coef * m[i].z;
-                    Tf += coef * m[i].w;
+                    const R coef = CoefGroup<R>::get(g[j / V], i);
+                    o.x += coef * m[i].x;
+                    o.y += coef * m[i].y;
+                    o.z += coef * m[i].z;
+                    o.w += coef * m[i].w;
                 }
             }
         }
-    }
+    };
+    v4 of;
+    rbf_sum(cf0, cf, of);
+    const R pf = of.x, uxf = of.y, uyf = of.z, Tf = of.w;
     gradient();
     const R gpx = quad_bcast<0>(gxk), gpy = quad_bcast<0>(gyk), guxx = quad_bcast<1>(gxk),
             guyx = quad_bcast<1>(gyk), guxy = quad_bcast<2>(gxk), guyy = quad_bcast<2>(gyk),
@@ -851,17 +855,14 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
         // or the unlimited linear state where the compact range is flat
         if constexpr (GP)
         for (int g = 0; g < p.ngp; ++g) {
-            auto atg = [&](int m) { return rbf_at(p.rbf_gp, p.rbfRow, c, g * maxC + k, p.ngp * maxC, m); };
-            R cg = atg(0);
-            R pg = cg * wc.x, uxg = cg * wc.y, uyg = cg * wc.z, Tg = cg * wc.w;
-            for (int ci = 0; ci < S; ++ci) {
-                const v4 wj = sW[sRows[lc * SW + ci]];
-                cg = atg(ci + 1);
-                pg += cg * wj.x;
-                uxg += cg * wj.y;
-                uyg += cg * wj.z;
-                Tg += cg * wj.w;
-            }
+            const R* ag = p.rbf_gp + (slice * p.ngp + g) * maxC * p.rbfRow;
+            cf0 = ag[a0];
+#pragma unroll
+            for (int i = 0; i < NG; ++i)
+                if (i * V < rows) cf[i] = (reinterpret_cast<const G*>(ag) + i * 64)[a1];
+            v4 q;
+            rbf_sum(cf0, cf, q);
+            const R pg = q.x, uxg = q.y, uyg = q.z, Tg = q.w;
             const v4 dg = p.fgd[(size_t)g * nf + f];
             const R gx = (R)(isNei ? dg.z : dg.x), gy = (R)(isNei ? dg.w : dg.y);
             v4 og;
