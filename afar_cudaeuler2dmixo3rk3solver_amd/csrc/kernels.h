@@ -22,92 +22,105 @@ template <> struct VT<float> {
 };
 
 // Everything a kernel reads or writes, passed by value.  Cell arrays hold nc
-// real cells followed (where noted) by nb boundary pseudo-cells.
+// real cells followed (where noted) by nb boundary pseudo-cells.  A kernel
+// waits for each 64-byte line of its arguments in turn, so the fields lie by
+// use: the counts fill the first line, the second and the start of the third
+// are the update's, the next the BVD's, the reconstruction's and the flux's
+// (back to back on 20k quads: update 4.9 us with its fields spread over five
+// lines, 4.4 so; BVD 4.1, 3.9; float flux with the CFL bound 7.0, 6.7).
 template <typename R>
 struct DevPtrs {
+    using v4 = typename VT<R>::v4;
+    using v2 = typename VT<R>::v2;
     int nc, nf, nb, maxS, maxC, ntiles;
+    int stenW;                 // ids per row of sten, a multiple of 8
+    int hfix, hcap;            // halo ids per row, capacity of the LDS halo (the dummy member follows it)
+    int rbfRow;                // elements of a row of coefficients
     int lds_sten_off;          // byte offset of the stencil ids in the reconstruction kernels' LDS
     int lds_m_off;             // byte offset of the tile's least-squares weights (four-lane kernel)
     int lds_bvd_sten_off;      // byte offset of the stencil ids in the BVD kernel's LDS
     int boundaryFirstOrder;    // extension: first-order faces in cells with a boundary face
-    typename VT<R>::v4* W;     // nc+nb primitive p, Ux, Uy, T
+    int storeFlat;             // the reconstruction stores what fflat lets it leave out, too
+    int ngp;                   // extension (faceQuadrature): flux points per internal face; 0: its centre only
+
+    v4* W;                     // nc+nb primitive p, Ux, Uy, T
+    const int32_t* slot_face;  // sliced ELL, +-(face+1)
+    const uint8_t* ccnt;       // nc compact stencil size
+    const uint8_t* scnt;       // nc stencil size
     double4* U;                // nc conserved rho, rhoUx, rhoUy, rhoE
     double4* Uold;             // nc
     const double* vol;         // nc
-    typename VT<R>::v2 *gp, *gu, *gv, *gT;  // nc: grad p; (dUx/dx, dUx/dy); (dUy/dx, dUy/dy); grad T
-    typename VT<R>::v4* lim;   // nc limiters p, Ux, Uy, T, then one entry of ones
+    const int32_t* cinst;      // nc instance of each cell, or nullptr (see ninst)
+
+    double4* flux;             // nf + nb face fluxes (FP32-mixed face-centre path: boundary faces only)
+    float4* flux32;            // FP32-mixed face-centre path: the nf internal faces' fluxes as computed,
+                               // in float (exact); else null
     int8_t* smooth;            // nc+nb smoothness flag (shockIndicator[2c])
+    int8_t* tlim;              // nc: BJ(raw T limiter) < VALID_LIM_FACTOR (the BVD test's limiter condition)
+    R* tTVD;                   // sliced ELL, the BVD test's limited linear temperature on the cell's face,
+                               // Tc + BJ(raw T limiter) * (grad T . d), formed by the reconstruction
+    R* fvT;                    // 2*nf face temperatures (see fv)
+    const uint16_t* sten;      // one row per cell: LDS-local stencil ids, then the dummy member's
+    const int32_t* halo;       // ntiles rows of hfix ids
+
+    const int32_t* more_ptr;   // ntiles+1, ids of the longer lists past their row
+    const int32_t* halo_more;
     int8_t* ftype;             // nc final reconstruction type (shockIndicator[2c+1])
-    uint8_t* flat_prev;        // nc: the cell took the flat branch at the last reconstruction
+    v4* lim;                   // nc limiters p, Ux, Uy, T, then one entry of ones
+    v2 *gp, *gu, *gv, *gT;     // nc: grad p; (dUx/dx, dUx/dy); (dUy/dx, dUy/dy); grad T
+
     // nf pairs (own, nei), face-centre path: that side's cell is flat, so its
     // face state is W + grad . d and its limiters 1; the face pass forms both
     // and the reconstruction stores neither (storeFlat: it stores them too).
     // Written only where a cell's branch changed.
     uint8_t* fflat;
-    int storeFlat;
-    const uint8_t* scnt;       // nc stencil size
-    const uint8_t* ccnt;       // nc compact stencil size
-    int stenW;                 // ids per row of sten, a multiple of 8
-    const uint16_t* sten;      // one row per cell: LDS-local stencil ids, then the dummy member's
-    const int32_t* slot_face;  // sliced ELL, +-(face+1)
-    const typename VT<R>::v2* slot_d;  // sliced ELL, face centre - cell centre, in the kernels' precision
-    const double2* slot_e;     // sliced ELL, compact neighbour - cell centre (K3 only)
+    uint8_t* flat_prev;        // nc: the cell took the flat branch at the last reconstruction
     // FP64 four-lane reconstruction: the slot geometry and least-squares
     // weights are formed from these instead of read from slot_d, slot_dr, lsq
-    const double2* cen;        // nc+nb cell and pseudo-cell centres
     const double2* fcen;       // nf+nb face centres
+    const double2* cen;        // nc+nb cell and pseudo-cell centres
     const double2* fshift;     // nf periodic shift of the neighbour centre, or null when every shift is zero
-    // Face-centre flux passes with the FP64 geometry (FP64; FP32-mixed with
-    // the CFL bound): the face's offsets from both cell centres (and the
-    // centre distance of the CFL bound) are formed from cen, fcen, fshift;
-    // the face area vector and its magnitude are read from these
-    const double2* fsf;        // nf Sf
-    const double* fmag;        // nf magSf
-    R* slot_dr;                // sliced ELL, |slot_e| in the kernels' precision (written by K3)
-    typename VT<R>::v2* lsq;   // sliced ELL, least-squares weights
-    int rbfRow;                // elements of a row of coefficients
-    const R* rbf;              // RBF coefficients: maxC rows per slice (DevLayout::rbf_at)
-    int hfix, hcap;            // halo ids per row, capacity of the LDS halo (the dummy member follows it)
-    const int32_t* halo;       // ntiles rows of hfix ids
-    const int32_t* more_ptr;   // ntiles+1, ids of the longer lists past their row
-    const int32_t* halo_more;
-    const int2* fcell;         // nf own, nei
-    const double4* fgeo;       // 2*nf: (Sfx, Sfy, magSf, deltaR), (dxo, dyo, dxn, dyn)
-    const float4* fgeo32;      // FP32-mixed: fgeo rounded to float (the flux pass without the CFL bound
-                               // uses the geometry in float only); else null
     // 2*nf reconstructed face values [2f + side].  FP64: one array per
     // variable (fvp, fvu, fvv, fvT; fv null).  FP32-mixed: (p, Ux, Uy, T)
     // records in fv and the temperatures again in fvT (fvp, fvu, fvv null):
     // 4-byte scattered stores into four arrays measured slower than one
     // 16-byte record.  The BVD test reads fvT alone.
-    typename VT<R>::v4* fv;
-    R *fvp, *fvu, *fvv, *fvT;
-    R* tTVD;                   // sliced ELL, the BVD test's limited linear temperature on the cell's face,
-                               // Tc + BJ(raw T limiter) * (grad T . d), formed by the reconstruction
-    int8_t* tlim;              // nc: BJ(raw T limiter) < VALID_LIM_FACTOR (the BVD test's limiter condition)
-    // extension (faceQuadrature): flux at ngp points per internal face
-    int ngp;                   // 0: face centre only (reference)
-    double gpw[4];             // point weights, sum 1
-    const R* rbf_gp;           // RBF coefficients at the points: ngp * maxC rows per slice
-    const typename VT<R>::v4* fgd;  // ngp*nf: point - owner centre (x, y), point - neighbour centre (z, w),
-                                    // in the kernels' precision
-    typename VT<R>::v4* fvg;   // ngp*2*nf reconstructed states at the points, [(g*nf + f)*2 + side]
-    double4* flux;             // nf + nb face fluxes (FP32-mixed face-centre path: boundary faces only)
-    float4* flux32;            // FP32-mixed face-centre path: the nf internal faces' fluxes as computed,
-                               // in float (exact); else null
+    R *fvp, *fvu, *fvv;
+
+    v4* fv;
+    const int2* fcell;         // nf own, nei
+    // Faces.  The CFL bound needs Sf, magSf and fcfl in double in either
+    // precision; the FP64 face-centre flux forms the face's offsets from both
+    // cell centres from cen, fcen, fshift; FP32-mixed reads its own records.
+    const double2* fsf;        // nf Sf
+    const double* fmag;        // nf magSf
+    const double2* fcfl;       // nf distance of the cell centres, the owner's share of it
+    const float4* fsf32;       // FP32-mixed: nf (Sfx, Sfy, magSf, 0) rounded to float; else null
+    const float4* foff32;      // FP32-mixed: nf (dxo, dyo, dxn, dyn) rounded to float; else null
+    double* dt_part;           // dt_cap partial minima of the CFL pass
+
+    const R* rbf;              // RBF coefficients: maxC rows per slice (DevLayout::rbf_at)
+    const v2* slot_d;          // sliced ELL, face centre - cell centre, in the kernels' precision
+    v2* lsq;                   // sliced ELL, least-squares weights
+    R* slot_dr;                // sliced ELL, |slot_e| in the kernels' precision (written by K3)
+    const double2* slot_e;     // sliced ELL, compact neighbour - cell centre (K3 only)
     const int32_t* bcell;      // nb
     const uint8_t* blabel;     // nb
     const double4* bgeo;       // nb (Sfx, Sfy, magSf, 0)
     const double4* bval;       // nb fixed values of label 6
+    // extension (faceQuadrature): flux at ngp points per internal face
+    double gpw[4];             // point weights, sum 1
+    const R* rbf_gp;           // RBF coefficients at the points: ngp * maxC rows per slice
+    const v4* fgd;             // ngp*nf: point - owner centre (x, y), point - neighbour centre (z, w),
+                               // in the kernels' precision
+    v4* fvg;                   // ngp*2*nf reconstructed states at the points, [(g*nf + f)*2 + side]
     double* dt;                // device time step of each instance (ninst)
-    double* dt_part;           // dt_cap partial minima of the CFL pass
     unsigned int* dt_count;    // tickets of the CFL pass: kCflGroups + 1 counters 128 bytes apart
     int dt_cap;                // capacity of dt_part: kCflBlocks or two per flux block, whichever is larger
     // Batches: ninst independent meshes stored one after the other (cells,
     // internal faces, boundary faces each contiguous per instance).  Each has
     // its own CFL time step.  A single mesh is ninst = 1 with cinst = nullptr.
     int ninst;
-    const int32_t* cinst;      // nc instance of each cell, or nullptr
     const int32_t* finst_off;  // ninst+1 first internal face of each instance
     // Device clock of each instance: tctl[4i] = t, tctl[4i+1] = end time,
     // tctl[4i+2] = steps taken.  The device time step is clipped to land on

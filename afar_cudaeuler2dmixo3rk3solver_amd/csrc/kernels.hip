@@ -90,6 +90,19 @@ __global__ void k_lsq(DevPtrs<R> p) {
     }
 }
 
+// The gas as the face passes use it: what every face would divide out for
+// itself is formed once on the host, with the kernels' expressions in the
+// precision they use it in (a float widened to double comes back exactly).
+struct GasArgs {
+    double R, Cv, CFL;
+    double gamma;  // (Cv + R) / Cv
+    double c2T;    // (R / Cv + 1) R, the CFL bound's
+    double Kd;     // KFVS: 2 Cv / R - 2
+};
+template <typename R> static inline GasArgs gas_args(double Rg, double Cv, double CFL) {
+    return {Rg, Cv, CFL, (Cv + Rg) / Cv, (Rg / Cv + 1.0) * Rg, (double)((R)2 * (R)Cv / (R)Rg - (R)2)};
+}
+
 // ---------------------------------------------------------------- K4 time step
 
 __device__ __forceinline__ double block_min_256(double v, double* wmin) {
@@ -107,32 +120,37 @@ __device__ __forceinline__ double block_min_256(double v, double* wmin) {
 }
 
 // Time-step bound of one internal face (cudaFieldOperation.h:124-180).
+// g: the distance of the two cell centres and the owner's share of it
+// (DevPtrs::fcfl); c2T: sound speed squared per unit of temperature.
 template <typename V4>
-__device__ __forceinline__ double cfl_face_dt(const double4& g0, const double4& g1, const V4& wo, const V4& wn,
-                                              double R_, double Cv, double CFL) {
-    const double Sfx = g0.x, Sfy = g0.y, magSf = g0.z, deltaR = g0.w;
-    const double fraction = afar_hypot(g1.x, g1.y) / deltaR;
+__device__ __forceinline__ double cfl_face_dt(double Sfx, double Sfy, double magSf, const double2& g, const V4& wo,
+                                              const V4& wn, double c2T, double CFL) {
+    const double deltaR = g.x, fraction = g.y;
     const double uxo = wo.y, uyo = wo.z, To = wo.w, uxn = wn.y, uyn = wn.z, Tn = wn.w;
     return CFL * deltaR * magSf /
            ((1.0 - fraction) * fabs(uxo * Sfx + uyo * Sfy) + fraction * fabs(uxn * Sfx + uyn * Sfy) +
-            sqrt((R_ / Cv + 1.0) * R_ * ((1.0 - fraction) * To + fraction * Tn)) * magSf);
+            sqrt(c2T * ((1.0 - fraction) * To + fraction * Tn)) * magSf);
 }
 
 // Each block reduces a contiguous chunk of faces (stride loop) to one
 // partial minimum; the last block to finish reduces the partials and stores
 // the time step on the device and, for the host that waits for it, in pinned
 // host memory.  Blocks draw tickets by group of kCflGroup, the last of each
-// group one more: 1024 tickets on one address take 20 us (250k quads 31 us a
-// launch), on 32 addresses next to nothing (XX us).
+// group one more: 1024 tickets on one address, each behind a fence that writes
+// the L2 back, took 20 us (250k quads 31 us a launch, so 11.5).  The centres'
+// distance and the owner's share of it are stored with the face (16 B) instead
+// of formed from its offsets (40 B, a root and a division): 11.5 -> 9.0 us,
+// 1.5M triangles 43 -> 30, 740k 24 -> 18.
 template <typename R>
-__global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double R_, double Cv, double CFL, int chunk, double* host_dt) {
+__global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double c2T, double CFL, int chunk, double* host_dt) {
     const int blk = xcd_tile(blockIdx.x, gridDim.x);
     const int f0 = blk * chunk;
     const int f1 = min(p.nf, f0 + chunk);
     double dtf = 1e5;
     for (int f = f0 + threadIdx.x; f < f1; f += 256) {
         const int2 oc = p.fcell[f];
-        const double d = cfl_face_dt(p.fgeo[2 * f], p.fgeo[2 * f + 1], p.W[oc.x], p.W[oc.y], R_, Cv, CFL);
+        const double2 sf = p.fsf[f];
+        const double d = cfl_face_dt(sf.x, sf.y, p.fmag[f], p.fcfl[f], p.W[oc.x], p.W[oc.y], c2T, CFL);
         dtf = d < dtf ? d : dtf;  // a NaN face value never replaces the minimum
     }
     __shared__ double wmin[4];
@@ -1107,7 +1125,7 @@ __device__ __forceinline__ R minimize_delta(R L, R Rv, R LT, R RT) {
 
 template <typename R>
 __device__ __forceinline__ void kfvs_flux(R& rhoFlux, R& rhoUxFlux, R& rhoUyFlux, R& rhoEFlux, R rhoL, R rhoR,
-                                          R pL, R pR, R uxL, R uxR, R uyL, R uyR, R TL, R TR, R Rg, R Cv, R magSf,
+                                          R pL, R pR, R uxL, R uxR, R uyL, R uyR, R TL, R TR, R Kd, R Cv, R magSf,
                                           R Sfx, R Sfy) {
     // cudaRiemannSolver.h:16-68
     const R nfx = Sfx / magSf, nfy = Sfy / magSf;
@@ -1126,7 +1144,6 @@ __device__ __forceinline__ void kfvs_flux(R& rhoFlux, R& rhoUxFlux, R& rhoUyFlux
     const R Mu2n = uxRl * Mu1n + (R)0.5 * Mu0n / lamR;
     const R Mu3n = uxRl * Mu2n + Mu1n / lamR;
     const R Mv1L = uyLl, Mv1R = uyRl;
-    const R Kd = (R)2 * Cv / Rg - (R)2;
     const R trho = rhoL * Mu1p + rhoR * Mu1n;
     const R trhoUx = rhoL * Mu2p + rhoR * Mu2n;
     const R trhoUy = rhoL * Mu1p * Mv1L + rhoR * Mu1n * Mv1R;
@@ -1162,15 +1179,23 @@ __device__ __forceinline__ void roe_flux(R& rhoFlux, R& rhoUxFlux, R& rhoUyFlux,
     const R r3 = (dP + rhoT * cT * dV) / ((R)2 * cT * cT);
     const R cL = sqrt(fmax((gamma - (R)1) * (hL - (R)0.5 * (uxL * uxL + uyL * uyL)), (R)1e-20));
     const R cR = sqrt(fmax((gamma - (R)1) * (hR - (R)0.5 * (uxR * uxR + uyR * uyR)), (R)1e-20));
-    R eps = (R)2 * fmax((R)0, (VR - cR) - (VL - cL));
-    R l1 = fabs(VT_ - cT);
-    l1 = (R)(l1 >= eps) * l1 + (R)(l1 < eps) * ((l1 * l1 + eps * eps) / ((R)2 * eps + (R)1e-30));
-    eps = (R)2 * fmax((R)0, VR - VL);
-    R l2 = fabs(VT_);
-    l2 = (R)(l2 >= eps) * l2 + (R)(l2 < eps) * ((l2 * l2 + eps * eps) / ((R)2 * eps + (R)1e-30));
-    eps = (R)2 * fmax((R)0, (VR + cR) - (VL + cL));
-    R l3 = fabs(VT_ + cT);
-    l3 = (R)(l3 >= eps) * l3 + (R)(l3 < eps) * ((l3 * l3 + eps * eps) / ((R)2 * eps + (R)1e-30));
+    // Harten's entropy fix, (l^2 + eps^2) / (2 eps + 1e-30) below eps.  At or
+    // above eps the reference's blend, 1 * l + 0 * quotient, is l itself as
+    // long as the quotient is finite, which it is below kMax (0 <= eps <= l):
+    // the three divisions are left to wavefronts with a face that needs one
+    // (of 17 on a Roe face; 740k cells in float 34.5 -> 32.5 us).
+    constexpr R kMax = sizeof(R) == 8 ? (R)1e100 : (R)1e4;
+    const R e1 = (R)2 * fmax((R)0, (VR - cR) - (VL - cL)), e2 = (R)2 * fmax((R)0, VR - VL),
+            e3 = (R)2 * fmax((R)0, (VR + cR) - (VL + cL));
+    R l1 = fabs(VT_ - cT), l2 = fabs(VT_), l3 = fabs(VT_ + cT);
+    if (!(l1 >= e1 && l2 >= e2 && l3 >= e3 && fmax(l1, l3) < kMax)) {
+        auto fix = [](R l, R e) {
+            return (R)(l >= e) * l + (R)(l < e) * ((l * l + e * e) / ((R)2 * e + (R)1e-30));
+        };
+        l1 = fix(l1, e1);
+        l2 = fix(l2, e2);
+        l3 = fix(l3, e3);
+    }
     rhoFlux -= (R)0.5 * (l1 * r1 + l2 * r2 + l3 * r3) * magSf;
     rhoUxFlux -= (R)0.5 * (l1 * r1 * (uxT - cT * nfx) + l2 * (r2 * uxT + rhoT * (dUx - dV * nfx)) + l3 * r3 * (uxT + cT * nfx)) * magSf;
     rhoUyFlux -= (R)0.5 * (l1 * r1 * (uyT - cT * nfy) + l2 * (r2 * uyT + rhoT * (dUy - dV * nfy)) + l3 * r3 * (uyT + cT * nfy)) * magSf;
@@ -1180,10 +1205,12 @@ __device__ __forceinline__ void roe_flux(R& rhoFlux, R& rhoUxFlux, R& rhoUyFlux,
 
 // Waves per SIMD the register allocator must allow for the face-centre flux
 // pass, per working type (build-time tuning knobs; 1 = no constraint).  The
-// FP64 passes take 104 VGPRs (4 waves) unconstrained.  At 5 waves the pass
-// without the CFL bound fits in 92 VGPRs without spills, yet measured 4%
-// slower per launch (the pass with it spills 20 bytes per lane); 6 and 8
-// waves spill (36 and 132 bytes per lane) and measured 26% and 108% slower.
+// FP64 passes take 128 VGPRs (4 waves) unconstrained, the float ones 63 and 70
+// (8 and 7 waves).  The FP64 pass with the CFL bound took 136 (3 waves) and 135
+// us on 1.5M cells while it formed the bound's distances itself; with them
+// stored, the gas constants from the host and the bound kept in LDS it has 4
+// waves: 120 us (without the bound 113 -> 108, entropy fix below).  At 5 waves
+// 44 and 61 VGPRs spill.
 #ifndef AFAR_FLUX_WPE_D
 #define AFAR_FLUX_WPE_D 1
 #endif
@@ -1203,14 +1230,17 @@ template <typename R, bool DT, bool GP> struct FluxWaves {
 // primitive state alone, which no kernel of the stage has changed yet.
 template <typename R, bool DT, bool GP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R, DT, GP>::value, 8))) void k_flux(
-    DevPtrs<R> p, double Rgas, double Cv, double CFL) {
+    DevPtrs<R> p, GasArgs gas) {
     using v4 = typename VT<R>::v4;
     using v2 = typename VT<R>::v2;
     constexpr bool FLAT = FormsFlat<R, GP>::value;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const int i = tile * 256 + threadIdx.x;
     const int nf = p.nf;
-    double dtf = 1e5;
+    // each face's bound waits in LDS for the reduction at the end: two
+    // registers fewer through the flux, which has none to spare for its waves
+    __shared__ double sDt[DT ? 256 : 1];
+    if (DT) sDt[threadIdx.x] = 1e5;
     if (i < nf) {
         const int f = i;
         const int2 oc = p.fcell[f];
@@ -1222,37 +1252,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
             skL = sk.x != 0;
             skR = sk.y != 0;
         }
-        double4 g0, g1;
-        if constexpr (sizeof(R) == 4 && !DT) {  // the geometry as the float arithmetic uses it
-            const float4 h0 = p.fgeo32[2 * f], h1 = p.fgeo32[2 * f + 1];
-            g0 = double4{h0.x, h0.y, h0.z, h0.w};
-            g1 = double4{h1.x, h1.y, h1.z, h1.w};
-        } else if constexpr (!GP) {
-            // the host layout's expressions in FP64: offsets of the face
-            // centre from the owner's centre and from the (shifted)
-            // neighbour's centre, and the distance between the two centres
-            // (FP32-mixed rounds the offsets to float below, as it rounds the
-            // stored record)
-            const double2 sf = p.fsf[f], fc = p.fcen[f], co = p.cen[own], cn = p.cen[nei];
-            const double2 fs = p.fshift ? p.fshift[f] : double2{0.0, 0.0};
-            const double xn = cn.x + fs.x, yn = cn.y + fs.y;
-            double dR = 0.0;
-            if (DT) {
-                const double ex = xn - co.x, ey = yn - co.y;
-                dR = afar_hypot(ex, ey);
-            }
-            g0 = double4{sf.x, sf.y, p.fmag[f], dR};
-            g1 = double4{fc.x - co.x, fc.y - co.y, fc.x - xn, fc.y - yn};
+        // The face's area vector, in double where the CFL bound needs it, and
+        // (at the face centre) its centre's offsets from the two cell centres:
+        // FP64 forms them with the host layout's expressions, the neighbour's
+        // centre shifted; FP32-mixed reads them rounded to float.
+        R magSf, Sfx, Sfy, dxL = 0, dyL = 0, dxR = 0, dyR = 0;
+        double2 sf{}, cg{};
+        double mag = 0.0;
+        if constexpr (sizeof(R) == 4 && !DT) {
+            const float4 s = p.fsf32[f];
+            Sfx = s.x;
+            Sfy = s.y;
+            magSf = s.z;
         } else {
-            g0 = p.fgeo[2 * f];
-            g1 = p.fgeo[2 * f + 1];
+            sf = p.fsf[f];
+            mag = p.fmag[f];
+            Sfx = (R)sf.x;
+            Sfy = (R)sf.y;
+            magSf = (R)mag;
         }
-        const R dxL = (R)g1.x, dyL = (R)g1.y, dxR = (R)g1.z, dyR = (R)g1.w;
+        if constexpr (DT) cg = p.fcfl[f];
+        if constexpr (!GP && sizeof(R) == 4) {
+            const float4 o = p.foff32[f];
+            dxL = o.x;
+            dyL = o.y;
+            dxR = o.z;
+            dyR = o.w;
+        } else if constexpr (!GP) {
+            const double2 fc = p.fcen[f], co = p.cen[own], cn = p.cen[nei];
+            const double2 fs = p.fshift ? p.fshift[f] : double2{0.0, 0.0};
+            dxL = (R)(fc.x - co.x);
+            dyL = (R)(fc.y - co.y);
+            dxR = (R)(fc.x - (cn.x + fs.x));
+            dyR = (R)(fc.y - (cn.y + fs.y));
+        }
         const int8_t to = p.ftype[own], tn = p.ftype[nei];
         const int isTVD_L = to != 0, isTVD_R = tn != 0;
         const int isShock = to < 0 || tn < 0;
-        const R magSf = (R)g0.z, Sfx = (R)g0.x, Sfy = (R)g0.y;
-        const R Rg = (R)Rgas;
+        const R Rg = (R)gas.R;
         const v4 wL = p.W[own], wR = p.W[nei];
         const v2 gpL = p.gp[own], gTL = p.gT[own];
         const v2 gpR = p.gp[nei], gTR = p.gT[nei];
@@ -1274,8 +1311,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
             }
         }
         if (DT) {
-            const double d = cfl_face_dt(g0, g1, wL, wR, Rgas, Cv, CFL);
-            dtf = d < dtf ? d : dtf;
+            const double d = cfl_face_dt(sf.x, sf.y, mag, cg, wL, wR, gas.c2T, gas.CFL);
+            sDt[threadIdx.x] = d < 1e5 ? d : 1e5;
         }
         const int shL = to < 0, shR = tn < 0;
         const v4 lL = face_limiters<R>(rL, shL);
@@ -1335,18 +1372,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
             const R dP = minimize_delta(pL, pR, pLT, pRT);
             const R dRho = minimize_delta(rhoL, rhoR, rhoLT, rhoRT);
 
-            const R CvR = (R)Cv;
+            const R CvR = (R)gas.Cv;
             R rhoFlux = (R)0.5 * rhoL * (uxL * Sfx + uyL * Sfy) + (R)0.5 * rhoR * (uxR * Sfx + uyR * Sfy);
             R rhoUxFlux = (R)0.5 * (rhoFlux * uxL + pL * Sfx) + (R)0.5 * (rhoFlux * uxR + pR * Sfx);
             R rhoUyFlux = (R)0.5 * (rhoFlux * uyL + pL * Sfy) + (R)0.5 * (rhoFlux * uyR + pR * Sfy);
             R rhoEFlux = (R)0.5 * rhoFlux * (CvR * TL + (R)0.5 * (uxL * uxL + uyL * uyL) + pL / rhoL) +
                          (R)0.5 * rhoFlux * (CvR * TR + (R)0.5 * (uxR * uxR + uyR * uyR) + pR / rhoR);
             if (isShock)
-                kfvs_flux<R>(rhoFlux, rhoUxFlux, rhoUyFlux, rhoEFlux, rhoL, rhoR, pL, pR, uxL, uxR, uyL, uyR, TL, TR, Rg,
-                             CvR, magSf, Sfx, Sfy);
+                kfvs_flux<R>(rhoFlux, rhoUxFlux, rhoUyFlux, rhoEFlux, rhoL, rhoR, pL, pR, uxL, uxR, uyL, uyR, TL, TR,
+                             (R)gas.Kd, CvR, magSf, Sfx, Sfy);
             else
                 roe_flux<R>(rhoFlux, rhoUxFlux, rhoUyFlux, rhoEFlux, rhoL, rhoR, pL, pR, uxL, uxR, uyL, uyR, TL, TR, dP,
-                            dRho, (R)((Cv + Rgas) / Cv), CvR, magSf, Sfx, Sfy);
+                            dRho, (R)gas.gamma, CvR, magSf, Sfx, Sfy);
             out0 = rhoFlux;
             out1 = rhoUxFlux;
             out2 = rhoUyFlux;
@@ -1386,10 +1423,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
         const double4 g = p.bgeo[b];
         const typename VT<R>::v4 w = p.W[p.nc + b];
         const double bp = w.x, bUx = w.y, bUy = w.z, bT = w.w;
-        const double rho = bp / (Rgas * bT);
+        const double rho = bp / (gas.R * bT);
         const double rhoFlux = rho * (bUx * g.x + bUy * g.y);
         p.flux[i] = double4{rhoFlux, rhoFlux * bUx + bp * g.x, rhoFlux * bUy + bp * g.y,
-                            rhoFlux * (Cv * bT + 0.5 * (bUx * bUx + bUy * bUy) + bp / rho)};
+                            rhoFlux * (gas.Cv * bT + 0.5 * (bUx * bUx + bUy * bUy) + bp / rho)};
     }
     if (DT) {
         // Two partials per tile of 256 faces: slot 0 for the instance of the
@@ -1399,6 +1436,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
         const int i0 = (p.cinst && nf > 0) ? p.cinst[p.fcell[f0].x] : 0;
         const int mine = (i < nf && p.cinst) ? p.cinst[p.fcell[i].x] : i0;
         __shared__ double wmin[4];
+        const double dtf = sDt[threadIdx.x];
         const double m0 = block_min_256(mine == i0 ? dtf : 1e5, wmin);
         const double m1 = block_min_256(mine == i0 ? 1e5 : dtf, wmin);
         if (threadIdx.x == 0) {
@@ -1653,7 +1691,7 @@ template <typename R>
 void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, double* host_dt, hipStream_t s) {
     const int nt = pad8(std::min(kCflBlocks, std::max(1, (p.nf + 255) / 256)));
     const int chunk = (p.nf + nt - 1) / nt;
-    hipLaunchKernelGGL(k_cfl<R>, dim3(nt), dim3(256), 0, s, p, Rg, Cv, CFL, chunk, host_dt);
+    hipLaunchKernelGGL(k_cfl<R>, dim3(nt), dim3(256), 0, s, p, gas_args<R>(Rg, Cv, CFL).c2T, CFL, chunk, host_dt);
 }
 
 template <typename R, bool GP, int MS>
@@ -1707,10 +1745,11 @@ int flux_blocks(int nf, int nb) { return pad8(std::max(1, (nf + nb + 255) / 256)
 
 template <typename R>
 void launch_flux(const DevPtrs<R>& p, double Rg, double Cv, hipStream_t s) {
+    const GasArgs gas = gas_args<R>(Rg, Cv, 0.0);
     if (p.ngp > 0)
-        hipLaunchKernelGGL((k_flux<R, false, true>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, Rg, Cv, 0.0);
+        hipLaunchKernelGGL((k_flux<R, false, true>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, gas);
     else
-        hipLaunchKernelGGL((k_flux<R, false, false>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, Rg, Cv, 0.0);
+        hipLaunchKernelGGL((k_flux<R, false, false>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, gas);
 }
 
 template <typename R>
@@ -1730,10 +1769,11 @@ void launch_residual_norm(const DevPtrs<R>& p, double* out, hipStream_t s) {
 
 template <typename R>
 void launch_flux_dt(const DevPtrs<R>& p, double Rg, double Cv, double CFL, hipStream_t s) {
+    const GasArgs gas = gas_args<R>(Rg, Cv, CFL);
     if (p.ngp > 0)
-        hipLaunchKernelGGL((k_flux<R, true, true>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, Rg, Cv, CFL);
+        hipLaunchKernelGGL((k_flux<R, true, true>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, gas);
     else
-        hipLaunchKernelGGL((k_flux<R, true, false>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, Rg, Cv, CFL);
+        hipLaunchKernelGGL((k_flux<R, true, false>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, gas);
 }
 
 template <typename R>

@@ -597,7 +597,8 @@ DevLayout make_dev_layout(const RefArrays& ra, int tile, int precision) {
 
     // internal faces
     L.fcell.resize(2 * (size_t)nf);
-    L.fgeo.resize(8 * (size_t)nf);
+    L.fcfl.resize(2 * (size_t)nf);
+    L.foff.resize(4 * (size_t)nf);
     parallel_for(nf, [&](int64_t f0, int64_t f1) {
         for (int64_t f = f0; f < f1; ++f) {
             const int own = ra.neighbour[2 * f], nei = ra.neighbour[2 * f + 1];
@@ -606,15 +607,13 @@ DevLayout make_dev_layout(const RefArrays& ra, int tile, int precision) {
             const double* F = &FACE[5 * f];
             const double xn = CELL[2 * nei] + FS[2 * f], yn = CELL[2 * nei + 1] + FS[2 * f + 1];
             const double ex = xn - CELL[2 * own], ey = yn - CELL[2 * own + 1];
-            double* g = &L.fgeo[8 * f];
-            g[0] = F[3];
-            g[1] = F[4];
-            g[2] = F[2];
-            g[3] = sqrt(ex * ex + ey * ey);
-            g[4] = F[0] - CELL[2 * own];
-            g[5] = F[1] - CELL[2 * own + 1];
-            g[6] = F[0] - xn;
-            g[7] = F[1] - yn;
+            double* g = &L.foff[4 * f];
+            g[0] = F[0] - CELL[2 * own];
+            g[1] = F[1] - CELL[2 * own + 1];
+            g[2] = F[0] - xn;
+            g[3] = F[1] - yn;
+            L.fcfl[2 * f] = sqrt(ex * ex + ey * ey);
+            L.fcfl[2 * f + 1] = sqrt(g[0] * g[0] + g[1] * g[1]) / L.fcfl[2 * f];
         }
     });
     // boundary faces

@@ -79,7 +79,8 @@ struct DevLayout {
     std::vector<int32_t> halo, more_ptr, halo_more;
     // per internal face
     std::vector<int32_t> fcell;           // 2*nf: own, nei
-    std::vector<double> fgeo;             // 8*nf: Sfx, Sfy, magSf, deltaR, dxo, dyo, dxn, dyn
+    std::vector<double> fcfl;             // 2*nf: distance of the cell centres, the owner's share of it
+    std::vector<double> foff;             // 4*nf: face centre - owner's, - neighbour's (shifted) centre
     // per boundary face
     std::vector<int32_t> bcell;           // nb
     std::vector<uint8_t> blabel;          // nb

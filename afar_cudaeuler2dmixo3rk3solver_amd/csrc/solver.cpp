@@ -738,10 +738,10 @@ class SolverImpl final : public DeviceSolver {
         P_.more_ptr = put(m_more_ptr, L_.more_ptr.data(), L_.more_ptr.size());
         P_.halo_more = put(m_halo_more, L_.halo_more.data(), L_.halo_more.size());
         P_.fcell = reinterpret_cast<const int2*>(put(m_fcell, L_.fcell.data(), 2 * nf));
-        P_.fgeo = reinterpret_cast<const double4*>(put(m_fgeo, L_.fgeo.data(), 8 * nf));
+        P_.fcfl = reinterpret_cast<const double2*>(put(m_fcfl, L_.fcfl.data(), 2 * nf));
         // Cell and face centres (and periodic shifts): the FP64 four-lane
-        // reconstruction forms its slot geometry from them, and the
-        // face-centre flux passes their offsets and the CFL bound's distance
+        // reconstruction forms its slot geometry from them, and the FP64
+        // face-centre flux passes their offsets
         P_.cen = P_.fcen = P_.fshift = nullptr;
         {
             P_.cen = reinterpret_cast<const double2*>(put(m_cen, ra_.CELL.data(), 2 * (nc + nb)));
@@ -755,10 +755,6 @@ class SolverImpl final : public DeviceSolver {
             for (double v : ra_.FSHIFT) shifted = shifted || v != 0.0 || std::signbit(v);  // -0.0 counts
             if (shifted) P_.fshift = reinterpret_cast<const double2*>(put(m_fshift, ra_.FSHIFT.data(), 2 * nf));
         }
-        // The face-centre flux passes that use the FP64 geometry (every FP64
-        // pass, the FP32-mixed pass with the CFL bound) form their offsets
-        // from the centres above and read Sf and magSf alone (40 instead of
-        // 64 B per face)
         P_.fsf = nullptr;
         P_.fmag = nullptr;
         {
@@ -771,11 +767,17 @@ class SolverImpl final : public DeviceSolver {
             P_.fsf = reinterpret_cast<const double2*>(put(m_fsf, sf.data(), sf.size()));
             P_.fmag = put(m_fmag, mag.data(), mag.size());
         }
-        P_.fgeo32 = nullptr;
+        P_.fsf32 = P_.foff32 = nullptr;
         if (sizeof(R) == 4) {
-            std::vector<float> g(L_.fgeo.size());
-            for (size_t i = 0; i < g.size(); ++i) g[i] = (float)L_.fgeo[i];
-            P_.fgeo32 = reinterpret_cast<const float4*>(put(m_fgeo32, g.data(), g.size()));
+            std::vector<float> s(4 * (size_t)nf), g(4 * (size_t)nf);
+            for (size_t i = 0; i < nf; ++i) {
+                s[4 * i] = (float)ra_.FACE[5 * i + 3];
+                s[4 * i + 1] = (float)ra_.FACE[5 * i + 4];
+                s[4 * i + 2] = (float)ra_.FACE[5 * i + 2];
+                for (int j = 0; j < 4; ++j) g[4 * i + j] = (float)L_.foff[4 * i + j];
+            }
+            P_.fsf32 = reinterpret_cast<const float4*>(put(m_fsf32, s.data(), s.size()));
+            P_.foff32 = reinterpret_cast<const float4*>(put(m_foff32, g.data(), g.size()));
         }
         P_.fv = nullptr;
         P_.fvp = P_.fvu = P_.fvv = nullptr;
@@ -857,7 +859,7 @@ class SolverImpl final : public DeviceSolver {
         synchronize();
         // the host keeps only what set_conserved needs (state, faces, boundary table)
         release_host(ra_.RBFbasis, ra_.RBFgp, ra_.stencil, ra_.cellFaces, ra_.neighbour, ra_.GPD);
-        release_host(L_.rbf, L_.rbf_gp, L_.slot_d, L_.slot_e, L_.fgeo, L_.fgd);
+        release_host(L_.rbf, L_.rbf_gp, L_.slot_d, L_.slot_e, L_.fcfl, L_.foff, L_.fgd);
         release_host(L_.sten, L_.slot_face, L_.fcell, L_.halo, L_.halo_more);
     }
 
@@ -884,7 +886,7 @@ class SolverImpl final : public DeviceSolver {
     int lanes_ = 1;  // threads per cell of the reconstruction kernel
     DevMem m_out_, m_flags_, m_stage_;  // output order (cell at each position), flags and states on their way out
     DevMem m_W, m_U, m_Uold, m_vol, m_gp, m_gu, m_gv, m_gT, m_lim, m_smooth, m_ftype, m_scnt, m_ccnt, m_sten,
-        m_slot_face, m_slot_d, m_slot_e, m_slot_dr, m_lsq, m_rbf, m_halo, m_more_ptr, m_halo_more, m_fcell, m_fgeo, m_fgeo32,
+        m_slot_face, m_slot_d, m_slot_e, m_slot_dr, m_lsq, m_rbf, m_halo, m_more_ptr, m_halo_more, m_fcell, m_fcfl, m_fsf32, m_foff32,
         m_fv, m_fvp, m_fvu, m_fvv, m_flux, m_flux32, m_bcell, m_blabel, m_bgeo, m_bval, m_dt, m_fvT, m_cinst, m_finst, m_tctl, m_res,
         m_rbf_gp, m_fgd, m_fvg, m_flat_prev, m_fflat, m_tlim, m_tTVD, m_cen, m_fcen, m_fshift, m_fsf, m_fmag;
 };

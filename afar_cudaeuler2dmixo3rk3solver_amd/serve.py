@@ -103,7 +103,7 @@ def footprint_bytes(mesh, precision):
     cell = nc * (4 * w * 4 + 32 * 3 + 8 + 4 * 2 * w + 2 + 2) + (nc + nb) * (4 * w + 1)
     slots = nslot * (2 * 1 + 4 + 16 + 16 + 2 * w + w) + ((nc + 63) // 64 * 64) * ((maxS + 7) // 8 * 8) * 2
     rbf = nslot * (maxS + 1) * w
-    faces = nf * (8 + 64 + 2 * 4 * w + 2) + (nf + nb) * 32 + nb * (4 + 1 + 64)
+    faces = nf * (8 + 16 + 2 * 4 * w + 2 + (32 if w == 4 else 0)) + (nf + nb) * 32 + nb * (4 + 1 + 64)
     # cell and face centres (the FP64 reconstruction, the face passes), the
     # periodic shifts (counted always: an upper bound), Sf and magSf
     centres = 16 * (nc + nb + nf + nb) + 16 * nf + 24 * nf
