@@ -21,6 +21,15 @@ template <> struct VT<float> {
     using v2 = float2;
 };
 
+// How a kernel's tiles are dealt to its blocks (xcd_tile): n tiles in 2^mlog
+// chunks, chunk j the tiles [j n / 2^mlog, (j + 1) n / 2^mlog), per the largest
+// chunk, magic = ceil(2^32 / per) or 0 for per = 1 (i / per without a division,
+// exact while i * per < 2^32).
+struct TileMap {
+    int n, per, mlog;
+    unsigned magic;
+};
+
 // Everything a kernel reads or writes, passed by value.  Cell arrays hold nc
 // real cells followed (where noted) by nb boundary pseudo-cells.  A kernel
 // waits for each 64-byte line of its arguments in turn, so the fields lie by
@@ -32,16 +41,16 @@ template <typename R>
 struct DevPtrs {
     using v4 = typename VT<R>::v4;
     using v2 = typename VT<R>::v2;
-    int nc, nf, nb, maxS, maxC, ntiles;
+    int nc, nf, nb, maxC;
+    TileMap map;               // of the kernel that is launched (set by the launchers)
     int stenW;                 // ids per row of sten, a multiple of 8
     int hfix, hcap;            // halo ids per row, capacity of the LDS halo (the dummy member follows it)
     int rbfRow;                // elements of a row of coefficients
     int lds_sten_off;          // byte offset of the stencil ids in the reconstruction kernels' LDS
     int lds_m_off;             // byte offset of the tile's least-squares weights (four-lane kernel)
     int lds_bvd_sten_off;      // byte offset of the stencil ids in the BVD kernel's LDS
-    int boundaryFirstOrder;    // extension: first-order faces in cells with a boundary face
-    int storeFlat;             // the reconstruction stores what fflat lets it leave out, too
-    int ngp;                   // extension (faceQuadrature): flux points per internal face; 0: its centre only
+    int16_t boundaryFirstOrder;  // extension: first-order faces in cells with a boundary face
+    int16_t storeFlat;         // the reconstruction stores what fflat lets it leave out, too
 
     v4* W;                     // nc+nb primitive p, Ux, Uy, T
     const int32_t* slot_face;  // sliced ELL, +-(face+1)
@@ -108,7 +117,9 @@ struct DevPtrs {
     const uint8_t* blabel;     // nb
     const double4* bgeo;       // nb (Sfx, Sfy, magSf, 0)
     const double4* bval;       // nb fixed values of label 6
+    int maxS, ntiles;
     // extension (faceQuadrature): flux at ngp points per internal face
+    int ngp;                   // 0: face centre only (reference)
     double gpw[4];             // point weights, sum 1
     const R* rbf_gp;           // RBF coefficients at the points: ngp * maxC rows per slice
     const v4* fgd;             // ngp*nf: point - owner centre (x, y), point - neighbour centre (z, w),
@@ -143,8 +154,8 @@ template <typename R> void launch_flux(const DevPtrs<R>& p, double Rg, double Cv
 // the step starts from) to per-block minima in p.dt_part; launch_dt_reduce
 // then stores their minimum in *p.dt.
 template <typename R> void launch_flux_dt(const DevPtrs<R>& p, double Rg, double Cv, double CFL, hipStream_t s);
-// Grid size of the flux kernels (blocks of 256 faces, a multiple of 8).
-int flux_blocks(int nf, int nb);
+// Tiles of the flux kernels (256 faces each).
+int flux_tiles(int nf, int nb);
 template <typename R> void launch_dt_reduce(const DevPtrs<R>& p, hipStream_t s);
 // Sum over cells of (density residual / volume)^2 from the current fluxes
 // into *out (device); res_part needs residual_blocks(nc) entries.

@@ -32,22 +32,23 @@ __device__ __forceinline__ size_t sell(int c, int k, int Kw) {
     return ((size_t)(c >> 6) * Kw + k) * 64 + (c & 63);
 }
 
-// Block -> tile mapping.  Blocks are dispatched round-robin over the 8 XCDs,
-// each with its own L2.  Each XCD takes chunks of XCD_CHUNK consecutive tiles
-// (cells in Hilbert order, so a chunk is a compact region whose halos are
-// mostly read through the same L2), and the 8 chunks running at a time are
-// neighbours in memory.  Measured on the 1.5M-cell bench: chunks of 16-64
-// tiles are 8% faster per step than one contiguous eighth of the grid per
-// XCD, and 4% faster than plain round-robin.  XCD_CHUNK is a build-time knob
-// (1: round-robin).
-#ifndef AFAR_XCD_CHUNK
-#define AFAR_XCD_CHUNK 32
-#endif
-__device__ __forceinline__ int xcd_tile(int b, int nblocks) {
-    constexpr int G = AFAR_XCD_CHUNK;
-    const int span = 8 * G;
-    if (b >= nblocks - nblocks % span) return b;  // the last partial span in dispatch order
-    return (b / span) * span + (b & 7) * G + (b >> 3) % G;
+// Block -> tile mapping (TileMap): the tile of this block, or -1.
+// Blocks are dispatched round-robin over the 8 XCDs, each with its own L2, and
+// what one kernel leaves in an L2 the next one finds there if the same XCD
+// works on the same cells.  Every kernel's tiles, whatever their size, are cut
+// into the same number of chunks (cells and faces lie in Hilbert order, so a
+// chunk is a compact region whose halos are mostly read through the same L2),
+// and chunk j is XCD j % 8's.  With chunks of 32 blocks of each kernel, 64 or
+// 256 cells a block, a cell's XCD changed from kernel to kernel: 20k quads 80.7
+// -> 73.1 us a step, in FP32-mixed 69.2 -> 65.8, 17k periodic quads 64.3 ->
+// 59.5, 134k triangles 170.6 -> 161.1, 48k in FP32-mixed 96.5 -> 89.9.
+__device__ __forceinline__ int xcd_tile(const TileMap& m) {
+    const unsigned b = blockIdx.x, i = b >> 3;
+    const unsigned q = m.magic ? __umulhi(i, m.magic) : i;  // i / per
+    const unsigned long long j = 8ull * q + (b & 7);        // the chunk
+    const int lo = (int)((j * m.n) >> m.mlog), hi = (int)(((j + 1) * m.n) >> m.mlog);
+    const int tile = lo + (int)(i - q * m.per);
+    return tile < hi ? tile : -1;
 }
 
 // exp and erfc of KFVS, both sides of a face at once: the library's own
@@ -143,9 +144,9 @@ __device__ __forceinline__ double cfl_face_dt(double Sfx, double Sfy, double mag
 // 1.5M triangles 43 -> 30, 740k 24 -> 18.
 template <typename R>
 __global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double c2T, double CFL, int chunk, double* host_dt) {
-    const int blk = xcd_tile(blockIdx.x, gridDim.x);
+    const int blk = xcd_tile(p.map);
     const int f0 = blk * chunk;
-    const int f1 = min(p.nf, f0 + chunk);
+    const int f1 = blk < 0 ? f0 : min(p.nf, f0 + chunk);
     double dtf = 1e5;
     for (int f = f0 + threadIdx.x; f < f1; f += 256) {
         const int2 oc = p.fcell[f];
@@ -267,8 +268,8 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
     using v2 = typename VT<R>::v2;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     v4* sW = reinterpret_cast<v4*>(smem_raw);
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    if (tile >= p.ntiles) return;
+    const int tile = xcd_tile(p.map);
+    if (tile < 0) return;
     const int tid = threadIdx.x, c = tile * TILE + tid;
     uint16_t* sRows = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
     if (c < p.nc) sW[tid] = p.W[c];
@@ -562,8 +563,8 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     uint16_t* sRows = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
     v2* sM = reinterpret_cast<v2*>(smem_raw + p.lds_m_off);            // 4 weights per cell
     double2* sC = reinterpret_cast<double2*>(smem_raw + p.lds_m_off);  // GEO: tile + halo centres instead
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    if (tile >= p.ntiles) return;
+    const int tile = xcd_tile(p.map);
+    if (tile < 0) return;
     const int t = threadIdx.x;
     const int lc = t >> 2, k = t & 3;
     const int c0 = tile * TILE, c = c0 + lc;
@@ -933,8 +934,8 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     int8_t* sS = reinterpret_cast<int8_t*>(smem_raw);
     uint16_t* sSt = reinterpret_cast<uint16_t*>(smem_raw + p.lds_bvd_sten_off);
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    if (tile >= p.ntiles) return;
+    const int tile = xcd_tile(p.map);
+    if (tile < 0) return;
     const int tid = threadIdx.x, c0 = tile * TILE, c = c0 + tid;
     const int maxC = p.maxC, nf = p.nf;
     const bool inb = c < p.nc;
@@ -1234,7 +1235,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FluxWaves<R
     using v4 = typename VT<R>::v4;
     using v2 = typename VT<R>::v2;
     constexpr bool FLAT = FormsFlat<R, GP>::value;
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = xcd_tile(p.map);
+    if (tile < 0) return;
     const int i = tile * 256 + threadIdx.x;
     const int nf = p.nf;
     // each face's bound waits in LDS for the reduction at the end: two
@@ -1556,7 +1558,8 @@ __device__ __forceinline__ double4 boundary_value(int label, double4 w, double4 
 template <typename R>
 __global__ __launch_bounds__(256) void k_update(DevPtrs<R> p, double Rgas, double gamma, double dt_val,
                                                  const double* dt_ptr, double b1, double b2, double b3, int last) {
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = xcd_tile(p.map);
+    if (tile < 0) return;
     const int c = tile * 256 + threadIdx.x;
     if (c >= p.nc) return;
     const int maxC = p.maxC, nf = p.nf;
@@ -1685,13 +1688,35 @@ void launch_lsq(const DevPtrs<R>& p, hipStream_t s) {
     hipLaunchKernelGGL(k_lsq<R>, dim3((p.nc + 255) / 256), dim3(256), 0, s, p);
 }
 
-static inline int pad8(int n) { return ((n + 7) / 8) * 8; }
+// p with the map of a kernel of n tiles (at most kCflBlocks in the CFL pass,
+// whose partials and tickets count the grid's blocks), and its grid: a block
+// per tile, rounded up to chunks of equal size.
+// 8 chunks at least, 128 at most, and between them the most that leave each
+// 2048 cells (FP64) or 4096 (FP32-mixed, half the bytes): smaller chunks leave
+// the XCDs evenly loaded where the flow is flat in part of the mesh (eighths:
+// 65k quads of a corner flow 102 -> 112 us a step, 260k 197 -> 228), more of
+// them than 128 break up the streams of the largest meshes (1.5M triangles
+// 1131 us with 128, 1154 with 512; with eighths 1237).
+template <typename R> static DevPtrs<R> mapped(const DevPtrs<R>& p, int n, unsigned& grid) {
+    static_assert(kCflBlocks % 128 == 0, "the CFL pass's grid stays within its blocks");
+    constexpr int kChunkCells = 16384 / sizeof(R);
+    int mlog = 3;
+    while (mlog < 7 && p.nc >> (mlog + 1) >= kChunkCells) ++mlog;
+    while (((unsigned long long)n * n) >> (mlog + 3) >= 1ull << 31) ++mlog;  // keeps i * per below 2^32
+    DevPtrs<R> q = p;
+    const unsigned per = std::max(1u, ((unsigned)n + (1u << mlog) - 1) >> mlog);
+    q.map = TileMap{n, (int)per, mlog, per == 1 ? 0u : 0xffffffffu / per + 1u};
+    grid = per << mlog;
+    return q;
+}
 
 template <typename R>
 void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, double* host_dt, hipStream_t s) {
-    const int nt = pad8(std::min(kCflBlocks, std::max(1, (p.nf + 255) / 256)));
+    const int nt = std::min(kCflBlocks, std::max(1, (p.nf + 255) / 256));
     const int chunk = (p.nf + nt - 1) / nt;
-    hipLaunchKernelGGL(k_cfl<R>, dim3(nt), dim3(256), 0, s, p, gas_args<R>(Rg, Cv, CFL).c2T, CFL, chunk, host_dt);
+    unsigned grid;
+    const DevPtrs<R> q = mapped(p, nt, grid);
+    hipLaunchKernelGGL(k_cfl<R>, dim3(grid), dim3(256), 0, s, q, gas_args<R>(Rg, Cv, CFL).c2T, CFL, chunk, host_dt);
 }
 
 template <typename R, bool GP, int MS>
@@ -1722,8 +1747,9 @@ void launch_reconstruct_t(const DevPtrs<R>& p, int nb, int tile, size_t lds, hip
 }
 
 template <typename R>
-void launch_reconstruct(const DevPtrs<R>& p, int tile, size_t lds, hipStream_t s, int lanes) {
-    const int nb = pad8(p.ntiles);
+void launch_reconstruct(const DevPtrs<R>& dev, int tile, size_t lds, hipStream_t s, int lanes) {
+    unsigned nb;
+    const DevPtrs<R> p = mapped(dev, dev.ntiles, nb);
     if (p.ngp > 0) {
         launch_reconstruct_t<R, true>(p, nb, tile, lds, s, lanes);
         return;
@@ -1732,8 +1758,9 @@ void launch_reconstruct(const DevPtrs<R>& p, int tile, size_t lds, hipStream_t s
 }
 
 template <typename R>
-void launch_bvd(const DevPtrs<R>& p, int tile, size_t lds, hipStream_t s) {
-    const int nb = pad8(p.ntiles);
+void launch_bvd(const DevPtrs<R>& dev, int tile, size_t lds, hipStream_t s) {
+    unsigned nb;
+    const DevPtrs<R> p = mapped(dev, dev.ntiles, nb);
     switch (tile) {
         case 64: hipLaunchKernelGGL((k_bvd<R, 64>), dim3(nb), dim3(64), lds, s, p); break;
         case 128: hipLaunchKernelGGL((k_bvd<R, 128>), dim3(nb), dim3(128), lds, s, p); break;
@@ -1741,15 +1768,17 @@ void launch_bvd(const DevPtrs<R>& p, int tile, size_t lds, hipStream_t s) {
     }
 }
 
-int flux_blocks(int nf, int nb) { return pad8(std::max(1, (nf + nb + 255) / 256)); }
+int flux_tiles(int nf, int nb) { return std::max(1, (nf + nb + 255) / 256); }
 
 template <typename R>
-void launch_flux(const DevPtrs<R>& p, double Rg, double Cv, hipStream_t s) {
+void launch_flux(const DevPtrs<R>& dev, double Rg, double Cv, hipStream_t s) {
+    unsigned grid;
+    const DevPtrs<R> p = mapped(dev, flux_tiles(dev.nf, dev.nb), grid);
     const GasArgs gas = gas_args<R>(Rg, Cv, 0.0);
     if (p.ngp > 0)
-        hipLaunchKernelGGL((k_flux<R, false, true>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, gas);
+        hipLaunchKernelGGL((k_flux<R, false, true>), dim3(grid), dim3(256), 0, s, p, gas);
     else
-        hipLaunchKernelGGL((k_flux<R, false, false>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, gas);
+        hipLaunchKernelGGL((k_flux<R, false, false>), dim3(grid), dim3(256), 0, s, p, gas);
 }
 
 template <typename R>
@@ -1768,19 +1797,22 @@ void launch_residual_norm(const DevPtrs<R>& p, double* out, hipStream_t s) {
 }
 
 template <typename R>
-void launch_flux_dt(const DevPtrs<R>& p, double Rg, double Cv, double CFL, hipStream_t s) {
+void launch_flux_dt(const DevPtrs<R>& dev, double Rg, double Cv, double CFL, hipStream_t s) {
+    unsigned grid;
+    const DevPtrs<R> p = mapped(dev, flux_tiles(dev.nf, dev.nb), grid);
     const GasArgs gas = gas_args<R>(Rg, Cv, CFL);
     if (p.ngp > 0)
-        hipLaunchKernelGGL((k_flux<R, true, true>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, gas);
+        hipLaunchKernelGGL((k_flux<R, true, true>), dim3(grid), dim3(256), 0, s, p, gas);
     else
-        hipLaunchKernelGGL((k_flux<R, true, false>), dim3(flux_blocks(p.nf, p.nb)), dim3(256), 0, s, p, gas);
+        hipLaunchKernelGGL((k_flux<R, true, false>), dim3(grid), dim3(256), 0, s, p, gas);
 }
 
 template <typename R>
 void launch_update(const DevPtrs<R>& p, double Rg, double gamma, double dt, const double* dt_ptr, double b1,
                    double b2, double b3, int last, hipStream_t s) {
-    const int nt = pad8(std::max(1, (p.nc + 255) / 256));
-    hipLaunchKernelGGL(k_update<R>, dim3(nt), dim3(256), 0, s, p, Rg, gamma, dt, dt_ptr, b1, b2, b3, last);
+    unsigned grid;
+    const DevPtrs<R> q = mapped(p, std::max(1, (p.nc + 255) / 256), grid);
+    hipLaunchKernelGGL(k_update<R>, dim3(grid), dim3(256), 0, s, q, Rg, gamma, dt, dt_ptr, b1, b2, b3, last);
 }
 
 template <typename R>

@@ -837,7 +837,7 @@ class SolverImpl final : public DeviceSolver {
         }
         dalloc(m_res, sizeof(double) * (residual_blocks(L_.nc) + 1));
         P_.res_part = m_res.as<double>();
-        const int dt_cap = std::max(kCflBlocks, 2 * flux_blocks(L_.nf, L_.nb));
+        const int dt_cap = std::max(kCflBlocks, 2 * flux_tiles(L_.nf, L_.nb));
         const size_t dt_bytes = (sizeof(double) * ni + 255) / 256 * 256;
         const size_t count_bytes = ((size_t)(kCflGroups + 1) * 128 + 255) / 256 * 256;
         dalloc(m_dt, dt_bytes + count_bytes + sizeof(double) * dt_cap);

@@ -1,0 +1,32 @@
+"""How a kernel's tiles are dealt to its blocks, over mesh sizes on both sides
+of the lines where the number of chunks changes, and below one tile a chunk.
+
+Two steps equal the oracle bit for bit (a tile left out or done by no block
+would leave its cells behind), with the time step of either entry point.
+"""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nx,ny,tile", [(7, 5, 64), (33, 31, 256), (127, 258, 64), (128, 256, 64), (257, 256, 128)])
+def test_every_tile_once(afar, nx, ny, tile, precision):
+    print("case: tile maps, %d x %d quads, tiles of %d, %s" % (nx, ny, tile, precision), flush=True)
+    from afar_cudaeuler2dmixo3rk3solver_amd import cases
+    mesh, W0 = cases.corner_case(nx=nx, ny=ny)
+    sc = afar.schemes(cOrder=5, fOrder=2, maxCo=0.3, precision=precision, tile=tile)
+    mesh.precompute(sc)
+    orc = O.OracleState(mesh.reference_arrays(sc, W0), sc.R, sc.Cv, mixed=precision == "mixed")
+    gpu = afar.BasicCUDASolver(mesh, sc, W0)
+    dt = gpu.set_delta_t()
+    assert dt == orc.adjust_time_step(sc.maxCo)
+    gpu.evolve(dt)
+    orc.evolve(dt)
+    gpu.evolve_auto(1)
+    orc.evolve(orc.adjust_time_step(sc.maxCo))
+    assert np.array_equal(gpu.conserved()[mesh.permutation()], orc.U)
+    gpu.close()
