@@ -76,13 +76,16 @@ struct DevPtrs {
     const int32_t* halo_more;
     int8_t* ftype;             // nc final reconstruction type (shockIndicator[2c+1])
     v4* lim;                   // nc limiters p, Ux, Uy, T, then one entry of ones
-    v2 *gp, *gu, *gv, *gT;     // nc: grad p; (dUx/dx, dUx/dy); (dUy/dx, dUy/dy); grad T
-
     // nf pairs (own, nei), face-centre path: that side's cell is flat, so its
-    // face state is W + grad . d and its limiters 1; the face pass forms both
-    // and the reconstruction stores neither (storeFlat: it stores them too).
-    // Written only where a cell's branch changed.
+    // face state is W + grad . d and its limiters 1; the face pass forms both,
+    // the BVD the temperatures it needs, and the reconstruction stores neither
+    // (storeFlat: it stores them too).  Written only where a cell's branch
+    // changed.
     uint8_t* fflat;
+    // nc: grad p; grad T; (dUx/dx, dUx/dy); (dUy/dx, dUy/dy)
+    v2 *gp, *gT, *gu;
+
+    v2* gv;
     uint8_t* flat_prev;        // nc: the cell took the flat branch at the last reconstruction
     // FP64 four-lane reconstruction: the slot geometry and least-squares
     // weights are formed from these instead of read from slot_d, slot_dr, lsq

@@ -248,14 +248,17 @@ template <typename R> __device__ __forceinline__ R to_venkat(R y) {
     return fmin((y * y + y + K<R>::VSMALL) / (y * y + (R)0.5 + (R)0.5 * y + K<R>::VSMALL), (R)1);
 }
 
-// Whether the face pass forms a flat cell's face states and limiters (FP64 at
-// the face centre): the reconstruction then writes 24 B per face side and 32 B
-// per cell less, and the face pass reads 64 B per face and 32 B per cell less,
-// where the gas is uniform, as ahead of every wave.  1.5M cells, 60% of them on
-// the full path: reconstruct 219 -> 192 us, flux 118 -> 114, step 1265 -> 1172;
-// nine corner flows 525 -> 480; 45k and 157k corner quads 105 -> 100, 167 ->
-// 159; 20k 83.6 -> 83.0; with no flat cell 67.9 -> 68.2.  FP32-mixed has half
-// the bytes to save and was slower for it (740k cells 469 -> 480).
+// Whether a flat cell's face states, limiters and BVD temperatures are formed
+// where they are read (FP64 at the face centre): the reconstruction then writes
+// 40 B per face side and 32 B per cell less, and the face pass reads 64 B per
+// face and 32 B per cell less, where the gas is uniform, as ahead of every
+// wave.  States and limiters, 1.5M cells, 60% of them on the full path:
+// reconstruct 219 -> 192 us, flux 118 -> 114, step 1265 -> 1172; nine corner
+// flows 525 -> 480; 20k quads 83.6 -> 83.0; with no flat cell 67.9 -> 68.2.  The
+// temperatures too: reconstruct 187 -> 177 us, BVD 18.2 -> 19.2 (it reads the
+// flags), step 1136 -> 1117, nine corner flows 456 -> 445, 250k quads 186 ->
+// 182; 20k quads and no flat cell 0.3 us longer.  FP32-mixed has half the bytes
+// to save and was slower for it (740k cells 469 -> 480).
 template <typename R, bool GP> struct FormsFlat {
     static constexpr bool value = sizeof(R) == 8 && !GP;
 };
@@ -352,15 +355,13 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
             if (f >= nf) continue;
             const v2 d = p.slot_d[sell(c, fi, maxC)];
             const R dx = d.x, dy = d.y;
+            if (!store) continue;
             v4 o;
             o.x = wc.x + gpx * dx + gpy * dy;
             o.y = wc.y + guxx * dx + guyx * dy;
             o.z = wc.z + guxy * dx + guyy * dy;
             o.w = wc.w + gTx * dx + gTy * dy;
-            if (store)
-                store_face_state(p, 2 * f + isNei, o);
-            else
-                p.fvT[2 * f + isNei] = o.w;
+            store_face_state(p, 2 * f + isNei, o);
             p.tTVD[sell(c, fi, maxC)] = wc.w + lT * (gTx * dx + gTy * dy);
             if constexpr (GP)
                 for (int g = 0; g < p.ngp; ++g) {  // flux points (extension): the same linear state there
@@ -784,17 +785,13 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
             (p.smooth + c0)[lc] = 0;
             (p.tlim + c0)[lc] = lT < K<R>::VALID_LIM_FACTOR;
         }
-        if (live) {
+        if (live && store) {
             v4 o;
+            o.x = wc.x + gpx * dx + gpy * dy;
+            o.y = wc.y + guxx * dx + guyx * dy;
+            o.z = wc.z + guxy * dx + guyy * dy;
             o.w = wc.w + gTx * dx + gTy * dy;
-            if (store) {
-                o.x = wc.x + gpx * dx + gpy * dy;
-                o.y = wc.y + guxx * dx + guyx * dy;
-                o.z = wc.z + guxy * dx + guyy * dy;
-                store_face_state(p, 2 * f + isNei, o);
-            } else {
-                p.fvT[2 * f + isNei] = o.w;
-            }
+            store_face_state(p, 2 * f + isNei, o);
             slots(p.tTVD)[row_k] = wc.w + lT * (gTx * dx + gTy * dy);
             if constexpr (GP)
                 for (int g = 0; g < p.ngp; ++g) {  // flux points (extension): the same linear state there
@@ -931,6 +928,7 @@ template <typename R, int TILE>
 __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
     using v4 = typename VT<R>::v4;
     constexpr int PF = 4;  // face slots whose data is requested in the first load rounds
+    constexpr bool FLAT = FormsFlat<R, false>::value;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     int8_t* sS = reinterpret_cast<int8_t*>(smem_raw);
     uint16_t* sSt = reinterpret_cast<uint16_t*>(smem_raw + p.lds_bvd_sten_off);
@@ -974,6 +972,7 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
     // them in a flagged tile for every cell, with the stencil block, measured
     // slower.)
     R tfo[PF], tfn[PF], tvd[PF];
+    unsigned short sks[PF];  // the face's flags of flat sides (DevPtrs::fflat)
     auto load_temps = [&](int fi) {
         const int sf = sfs[fi];
         const int f = (sf < 0 ? -sf : sf) - 1;
@@ -981,11 +980,13 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
             tfo[fi] = p.fvT[2 * f];
             tfn[fi] = p.fvT[2 * f + 1];
             tvd[fi] = (p.tTVD + slot0 + fi * 64)[cl];
+            if (FLAT) sks[fi] = reinterpret_cast<const unsigned short*>(p.fflat)[f];
         }
     };
 #pragma unroll
     for (int fi = 0; fi < PF; ++fi) {
         tfo[fi] = tfn[fi] = tvd[fi] = (R)0;
+        sks[fi] = 0;
         if (limited) load_temps(fi);
     }
     if (inb) sS[tid] = own;
@@ -1042,6 +1043,31 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
 #pragma unroll
         for (int fi = 0; fi < PF; ++fi) load_temps(fi);
     }
+    // The temperatures of a flat side, which are not stored, with the
+    // reconstruction's operations: seldom a limited cell's own, more often its
+    // neighbour's.
+    auto form_flat = [&](int sf, unsigned sk, R& TfOwn, R& TfNei, R& Tf_cur_TVD) {
+        const int f = (sf < 0 ? -sf : sf) - 1;
+        const int2 oc = p.fcell[f];
+        const double2 fc = p.fcen[f], fs = p.fshift ? p.fshift[f] : double2{0.0, 0.0};
+        auto form = [&](bool nei, R& Tf) {
+            const int s = nei ? oc.y : oc.x;
+            const double2 cs = p.cen[s];
+            const typename VT<R>::v2 g = p.gT[s];
+            const R T = p.W[s].w;
+            const R dx = (R)(fc.x - (nei ? cs.x + fs.x : cs.x)), dy = (R)(fc.y - (nei ? cs.y + fs.y : cs.y));
+            Tf = T + g.x * dx + g.y * dy;
+            if (nei == sf < 0) Tf_cur_TVD = T + (g.x * dx + g.y * dy);
+        };
+        if (sk & 0xff) form(false, TfOwn);
+        if (sk >> 8) form(true, TfNei);
+    };
+    if (FLAT && __builtin_expect((sks[0] | sks[1] | sks[2] | sks[3]) != 0, 0)) {
+        static_assert(PF == 4, "the flags of all slots read ahead");
+#pragma unroll
+        for (int fi = 0; fi < PF; ++fi)
+            if (sks[fi]) form_flat(sfs[fi], sks[fi], tfo[fi], tfn[fi], tvd[fi]);
+    }
     auto face = [&](int sf, R TfOwn, R TfNei, R Tf_cur_TVD) {
         const int isNei = sf < 0;
         const R Tf_cur = (R)isNei * TfNei + (R)(1 - isNei) * TfOwn;
@@ -1066,8 +1092,12 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
         const int f = (sf < 0 ? -sf : sf) - 1;
         if (f >= nf)
             bfaces += 1;
-        else if (isLimited)
-            face(sf, p.fvT[2 * f], p.fvT[2 * f + 1], (p.tTVD + slot0 + fi * 64)[cl]);
+        else if (isLimited) {
+            R To = p.fvT[2 * f], Tn = p.fvT[2 * f + 1], Tt = (p.tTVD + slot0 + fi * 64)[cl];
+            const unsigned sk = FLAT ? reinterpret_cast<const unsigned short*>(p.fflat)[f] : 0;
+            if (FLAT && sk) form_flat(sf, sk, To, Tn, Tt);
+            face(sf, To, Tn, Tt);
+        }
     }
     if (bfaces >= 2) bvd = 1;  // corner cells use the second-order reconstruction
     int finalType = (shockType > 0) * (shockTypeExt > 1) * (-2) + (bvd > 0);
