@@ -816,9 +816,9 @@ class SolverImpl final : public DeviceSolver {
         P_.blabel = put(m_blabel, L_.blabel.data(), nb);
         P_.bgeo = reinterpret_cast<const double4*>(put(m_bgeo, L_.bgeo.data(), 4 * nb));
         P_.bval = reinterpret_cast<const double4*>(put(m_bval, L_.bval.data(), 4 * nb));
-        // per-instance time steps, the ticket counter (own 256-byte line) and
-        // the CFL partials (two per flux tile, or kCflBlocks for the
-        // standalone pass)
+        // per-instance time steps, the standalone CFL pass's ticket counters
+        // and the CFL partials (two per flux tile, or kCflBlocks for that
+        // pass)
         const int ni = bi_.ninst();
         P_.ninst = ni;
         if (ni > 1) {

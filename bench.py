@@ -83,7 +83,10 @@ def kernel_bytes(st, w=8, ngp=0, geo=False):
     (slot_d) and distances are stored in the kernels' precision.  geo (the
     FP64 four-lane kernel at the face centre): instead of the face offsets,
     distances and least-squares weights it reads the cell and pseudo-cell
-    centres and, per compact slot, the face centre (16 B each).  ngp > 0
+    centres and, per compact slot, the face centre (16 B each).  FP64 at the
+    face centre stores face states, limiters and BVD temperatures of cells on
+    the full path only, marks the other sides (1 B, written on change), and the
+    flux and the BVD read what is stored.  ngp > 0
     (flux quadrature points): the reconstruction also reads each point's
     coefficients (full path) and offsets and writes each point's states; the
     flux reads those states and offsets instead of the face-centre states."""
@@ -91,39 +94,38 @@ def kernel_bytes(st, w=8, ngp=0, geo=False):
     sR, sfull = st["sum_int_coef_full"], st["int_slots_full"]
     ns = 2 * nf  # internal face slots
     slot_geo = 16 * (nc + nb) + 16 * sC if geo else 2 * w * ns + w * sfull + 2 * w * sC
+    cg = w == 8 and not ngp
+    nstored, sstored = (st["full_cells"], sfull) if cg else (nc, ns)  # cells, face sides
     # writes: gradients 8w, limiters 4w, smoothness flag and limiter condition per cell; O3 face state 4w
     # (FP64: one array per variable, the temperatures being what the BVD test reads; FP32: records and the
     # temperatures again, w) and the BVD test's limited linear temperature w per internal face side
     recon = (4 * w * (nc + nb) + 2 * nc + 2 * sS + 4 * sC + slot_geo + w * sR
-             + 8 * w * nc + 4 * w * nc + 2 * nc + 4 * w * ns + w * ns + (w * ns if w == 4 else 0))
+             + 8 * w * nc + 4 * w * nstored + 2 * nc + 4 * w * sstored + w * sstored + (w * ns if w == 4 else 0))
     # bvd reads flags, counts, stencil ids, face slots, both sides' O3 face temperatures and this side's
     # limited linear one, the limiter condition; writes the types (the face pass applies the limiter transform)
-    bvd = ((nc + nb) + 2 * nc + 2 * sS + 4 * sC + w * ns + w * ns + nc + nc)
-    # FP32-mixed: internal fluxes at the face centre are stored as floats, and
-    # the flux pass without the CFL bound reads the face geometry in float.
-    # FP64 at the face centre: both passes read Sf, magSf and the face centre
-    # (40 B per face) and the cells' centres (16 B per cell; a periodic mesh
-    # adds its 16-B shift per face), and form the offsets and the distance;
-    # so does the FP32-mixed pass with the CFL bound
+    bvd = ((nc + nb) + 2 * nc + 2 * sS + 4 * sC + w * sstored + w * sstored + (2 * nf if cg else 0) + nc + nc)
+    # Face geometry.  FP64: Sf, magSf and (at the face centre) the centre, 40 B
+    # per face, and the cells' centres, 16 B per cell (a periodic mesh adds its
+    # 16-B shift per face); FP32-mixed: Sf, magSf and the offsets as floats, 32
+    # B.  The CFL bound takes Sf, magSf and the centres' distance and share in
+    # FP64, 40 B.  At flux points no pass reads centres or offsets.  FP32-mixed
+    # stores the internal fluxes at the face centre as floats.
     fw = 4 * w if (w == 4 and not ngp) else 32
-    cg = w == 8 and not ngp
-    if cg:
-        dt_extra = 0
-    elif not ngp:
-        dt_extra = (40 - 8 * w) * nf + 16 * nc
-    else:  # flux points: the 64-B FP64 record
-        dt_extra = (64 - 8 * w) * nf
-    geo = 40 if cg else 8 * w
-    flux = (8 * nf + geo * nf + 8 * w * nf + nc * (4 * w + 4 * w + 8 * w + 1 + (16 if cg else 0)) + 32 * nb
+    if w == 8:
+        geo, dt_extra = (24 if ngp else 40), 16 * nf
+    else:
+        geo, dt_extra = (16 if ngp else 32), 24 * nf
+    flux = (8 * nf + geo * nf + 4 * w * sstored + (2 * nf if cg else 0)
+            + nc * (4 * w + 8 * w + 1 + (16 if cg else 0)) + 4 * w * nstored + 32 * nb
             + 4 * w * nb + fw * nf + 32 * nb)
     # U and Uold are read in the second and third stages, Uold alone in the first; the first two stages
     # write U, the last writes Uold only
     update = nc + 4 * sC + fw * nf + 32 * nb + 32 * nc * 5 / 3 + 8 * nc + 65 * nb + 32 * nc + 4 * w * (nc + nb)
-    cfl = 8 * nf + 48 * nf + 4 * w * nc
+    cfl = 8 * nf + 40 * nf + 4 * w * nc
     if ngp:
         recon += ngp * (w * sR + 4 * w * ns + 4 * w * ns)
         flux += ngp * (8 * w + 4 * w) * nf - 8 * w * nf
-    nblk = 8 * (((nf + nb + 255) // 256 + 7) // 8)  # flux grid: one CFL partial per block
+    nblk = (nf + nb + 255) // 256  # flux tiles: one CFL partial each
     return dict(cfl=cfl, reconstruct=recon, bvd=bvd, flux=flux, update=update,
                 flux_dt=flux + dt_extra + 8 * nblk, dt_reduce=8 * nblk)
 
