@@ -1718,21 +1718,24 @@ void launch_lsq(const DevPtrs<R>& p, hipStream_t s) {
     hipLaunchKernelGGL(k_lsq<R>, dim3((p.nc + 255) / 256), dim3(256), 0, s, p);
 }
 
-// p with the map of a kernel of n tiles (at most kCflBlocks in the CFL pass,
-// whose partials and tickets count the grid's blocks), and its grid: a block
-// per tile, rounded up to chunks of equal size.
+// p with the map of a kernel of n tiles and its grid: a block per tile, rounded
+// up to chunks of equal size.  maxLog: the most chunks (the CFL pass, whose
+// partials and tickets count the grid's blocks).
 // 8 chunks at least, 128 at most, and between them the most that leave each
 // 2048 cells (FP64) or 4096 (FP32-mixed, half the bytes): smaller chunks leave
 // the XCDs evenly loaded where the flow is flat in part of the mesh (eighths:
 // 65k quads of a corner flow 102 -> 112 us a step, 260k 197 -> 228), more of
 // them than 128 break up the streams of the largest meshes (1.5M triangles
-// 1131 us with 128, 1154 with 512; with eighths 1237).
-template <typename R> static DevPtrs<R> mapped(const DevPtrs<R>& p, int n, unsigned& grid) {
-    static_assert(kCflBlocks % 128 == 0, "the CFL pass's grid stays within its blocks");
-    constexpr int kChunkCells = 16384 / sizeof(R);
+// 1131 us with 128, 1154 with 512; with eighths 1237).  Past 128 a chunk holds
+// at most 12288 cells: 256 FP32-mixed corner flows, 8.2M cells in the largest
+// bucket, 7.54 -> 7.41 ms a step.
+template <typename R>
+static DevPtrs<R> mapped(const DevPtrs<R>& p, int n, unsigned& grid, int maxLog = 24) {
+    constexpr int kChunkCells = 16384 / sizeof(R), kMaxChunkCells = 12288;
     int mlog = 3;
     while (mlog < 7 && p.nc >> (mlog + 1) >= kChunkCells) ++mlog;
-    while (((unsigned long long)n * n) >> (mlog + 3) >= 1ull << 31) ++mlog;  // keeps i * per below 2^32
+    while (mlog < maxLog && p.nc >> mlog > kMaxChunkCells) ++mlog;
+    while (mlog < maxLog && ((unsigned long long)n * n) >> (mlog + 3) >= 1ull << 31) ++mlog;  // keeps i * per below 2^32
     DevPtrs<R> q = p;
     const unsigned per = std::max(1u, ((unsigned)n + (1u << mlog) - 1) >> mlog);
     q.map = TileMap{n, (int)per, mlog, per == 1 ? 0u : 0xffffffffu / per + 1u};
@@ -1745,7 +1748,8 @@ void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, double* h
     const int nt = std::min(kCflBlocks, std::max(1, (p.nf + 255) / 256));
     const int chunk = (p.nf + nt - 1) / nt;
     unsigned grid;
-    const DevPtrs<R> q = mapped(p, nt, grid);
+    static_assert(kCflBlocks == 1 << 10, "a tile per block and no more chunks than blocks");
+    const DevPtrs<R> q = mapped(p, nt, grid, 10);
     hipLaunchKernelGGL(k_cfl<R>, dim3(grid), dim3(256), 0, s, q, gas_args<R>(Rg, Cv, CFL).c2T, CFL, chunk, host_dt);
 }
 

@@ -15,6 +15,14 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("nx,ny,tile", [(7, 5, 64), (33, 31, 256), (127, 258, 64), (128, 256, 64), (257, 256, 128)])
 def test_every_tile_once(afar, nx, ny, tile, precision):
+    _two_steps(afar, nx, ny, tile, precision)
+
+
+def test_more_than_128_chunks(afar):
+    _two_steps(afar, 1300, 1250, 64, "fp64")
+
+
+def _two_steps(afar, nx, ny, tile, precision):
     print("case: tile maps, %d x %d quads, tiles of %d, %s" % (nx, ny, tile, precision), flush=True)
     from afar_cudaeuler2dmixo3rk3solver_amd import cases
     mesh, W0 = cases.corner_case(nx=nx, ny=ny)
