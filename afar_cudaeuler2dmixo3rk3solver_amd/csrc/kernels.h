@@ -53,7 +53,7 @@ struct DevPtrs {
     int16_t storeFlat;         // the reconstruction stores what fflat lets it leave out, too
 
     v4* W;                     // nc+nb primitive p, Ux, Uy, T
-    const int32_t* slot_face;  // sliced ELL, +-(face+1)
+    const int32_t* slot_face;  // sliced ELL, +-(face+1), slices of whole tiles
     const uint8_t* ccnt;       // nc compact stencil size
     const uint8_t* scnt;       // nc stencil size
     double4* U;                // nc conserved rho, rhoUx, rhoUy, rhoE

@@ -950,7 +950,8 @@ __global__ __launch_bounds__(TILE) void k_bvd(DevPtrs<R> p) {
     const int S = (p.scnt + c0)[cc], C = inb ? (int)(p.ccnt + c0)[cc] : 0;
     const int8_t own = (p.smooth + c0)[cc];
     const int limited = (p.tlim + c0)[cc];
-    // a wavefront's cells are one slice of the slot arrays
+    // A wavefront's cells are one slice of the slot arrays; slot_face has a slice
+    // of no slots for the wavefronts of the last tile past the last cell.
     const size_t slot0 = (size_t)((unsigned)(c0 + 64 * __builtin_amdgcn_readfirstlane(tid >> 6)) >> 6) * maxC * 64;
     const unsigned cl = tid & 63;
     int sfs[PF];

@@ -473,7 +473,9 @@ DevLayout make_dev_layout(const RefArrays& ra, int tile, int precision) {
     L.ccnt = ra.compactStencilSize;
     L.stenW = std::max(8, (maxS + 7) & ~7);
     L.sten.assign((size_t)L.nwaves * 64 * L.stenW, 0);
-    L.slot_face.assign(nslot, 0);
+    // a slice for every wavefront of the last tile, also past the last cell: the
+    // BVD pass reads a wavefront's slots before it knows which cells exist
+    L.slot_face.assign((size_t)L.ntiles * (tile / 64) * maxC * 64, 0);
     L.slot_d.assign(2 * nslot, 0.0);
     L.slot_e.assign(2 * nslot, 0.0);
     // Coefficients past a cell's stencil are -0.0 and their ids name a dummy member of

@@ -62,7 +62,7 @@ struct DevLayout {
     int stenW = 8;                        // ids per row of sten: maxS rounded up to whole 16-byte words
     std::vector<uint16_t> sten;           // nwaves*64*stenW, one row per cell: LDS-local ids, then the tile's
                                           // dummy member (tile + hcap)
-    std::vector<int32_t> slot_face;       // nwaves*maxC*64, +-(f+1), 0 = padding
+    std::vector<int32_t> slot_face;       // +-(f+1), 0 = padding; slices of whole tiles (nwaves or a few more)
     std::vector<double> slot_d;           // 2 per slot: face centre - cell centre
     std::vector<double> slot_e;           // 2 per slot: compact neighbour - cell centre
     // RBF coefficients of a slot (rbf_row(): rbfRow elements): the cell's own

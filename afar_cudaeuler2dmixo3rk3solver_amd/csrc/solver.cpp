@@ -723,7 +723,7 @@ class SolverImpl final : public DeviceSolver {
         P_.scnt = put(m_scnt, L_.scnt.data(), nc);
         P_.ccnt = put(m_ccnt, L_.ccnt.data(), nc);
         P_.sten = put(m_sten, L_.sten.data(), L_.sten.size());
-        P_.slot_face = put(m_slot_face, L_.slot_face.data(), nslot);
+        P_.slot_face = put(m_slot_face, L_.slot_face.data(), L_.slot_face.size());
         // face offsets in the kernels' precision (they use them in it only)
         P_.slot_d = reinterpret_cast<const v2*>(put_as_R(m_slot_d, L_.slot_d.data(), 2 * nslot));
         P_.slot_e = reinterpret_cast<const double2*>(put(m_slot_e, L_.slot_e.data(), 2 * nslot));
