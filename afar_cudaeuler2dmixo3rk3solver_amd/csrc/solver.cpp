@@ -8,8 +8,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
-#include <string>
 #include <mutex>
+#include <string>
+#include <utility>
+#include <vector>
 
 #include "kernels.h"
 
@@ -50,16 +52,54 @@ struct DevMem {
     template <typename T> T* as() const { return reinterpret_cast<T*>(p); }
 };
 
-// One double of pinned host memory, and its device address.
-struct PinnedDouble {
+// One double of pinned host memory and its device address, for a solver's host
+// time step.  hipHostFree waits for the whole device, so the doubles are slots
+// of pages that are kept until the process ends: a destroyed solver's slot goes
+// to the next one, and there are as many pages as the most solvers that lived
+// at one time need (a page holds kSlots, 64 bytes apart).
+class PinnedDouble {
+   public:
     double *p = nullptr, *dev = nullptr;
+    PinnedDouble() = default;
+    PinnedDouble(const PinnedDouble&) = delete;
+    PinnedDouble& operator=(const PinnedDouble&) = delete;
+    // the owner has waited for the last kernel that stores to the slot
     ~PinnedDouble() {
-        if (p) (void)hipHostFree(p);
+        if (!p) return;
+        Pool& pool = the_pool();
+        std::lock_guard<std::mutex> lk(pool.m);
+        pool.free.push_back({p, dev});
     }
     void alloc() {
-        check_hip(hipHostMalloc((void**)&p, sizeof(double), hipHostMallocMapped | hipHostMallocCoherent),
-                  "hipHostMalloc");
-        check_hip(hipHostGetDevicePointer((void**)&dev, p, 0), "hipHostGetDevicePointer");
+        Pool& pool = the_pool();
+        std::lock_guard<std::mutex> lk(pool.m);
+        if (pool.free.empty()) {
+            char *h = nullptr, *d = nullptr;
+            pool.free.reserve(kSlots * (pool.pages + 1));  // the destructor's push_back never allocates
+            check_hip(hipHostMalloc((void**)&h, 64 * kSlots,
+                                    hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable),
+                      "hipHostMalloc");
+            check_hip(hipHostGetDevicePointer((void**)&d, h, 0), "hipHostGetDevicePointer");
+            ++pool.pages;
+            for (size_t i = kSlots; i-- > 0;)
+                pool.free.push_back({reinterpret_cast<double*>(h + 64 * i), reinterpret_cast<double*>(d + 64 * i)});
+        }
+        p = pool.free.back().first;
+        dev = pool.free.back().second;
+        pool.free.pop_back();
+    }
+
+   private:
+    static constexpr size_t kSlots = 64;
+    struct Pool {
+        std::mutex m;
+        std::vector<std::pair<double*, double*>> free;  // host and device address
+        size_t pages = 0;
+    };
+    // never destroyed: solvers may outlive the library's static objects
+    static Pool& the_pool() {
+        static Pool* pool = new Pool;
+        return *pool;
     }
 };
 
@@ -869,7 +909,7 @@ class SolverImpl final : public DeviceSolver {
     BatchIndex bi_;
     DevLayout L_;
     DevPtrs<R> P_{};
-    PinnedDouble host_dt_;  // before the stream: freed after its last kernel
+    PinnedDouble host_dt_;  // before the stream: given back after its last kernel
     StreamHolder sh_;  // before the buffers: destroyed after them
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
