@@ -275,7 +275,7 @@ class SolverImpl final : public DeviceSolver {
 
     void read_conserved(int o0, int n, double* U) override {
         if (o0 < 0 || n < 0 || o0 + n > L_.nc) throw Error(1, "cell range out of bounds");
-        double4* st = staging();
+        double4* st = m_stage_.as<double4>();
         launch_gather_state(state_U(), m_out_.as<const int32_t>() + o0, st, n, stream_);
         check_hip(hipGetLastError(), "gather");
         touch(U, sizeof(double4) * n);
@@ -285,7 +285,7 @@ class SolverImpl final : public DeviceSolver {
 
     void read_fields(int o0, int n, double* W, int8_t* flags, bool pairs) override {
         if (o0 < 0 || n < 0 || o0 + n > L_.nc) throw Error(1, "cell range out of bounds");
-        double4* st = staging();
+        double4* st = m_stage_.as<double4>();
         int8_t* fl = m_flags_.as<int8_t>();
         launch_gather_fields<R>(P_, m_out_.as<const int32_t>() + o0, st, fl, pairs, n, stream_);
         check_hip(hipGetLastError(), "gather");
@@ -315,6 +315,9 @@ class SolverImpl final : public DeviceSolver {
         for (int c = 0; c < L_.nc; ++c) idx[out_pos ? out_pos[c] : c] = c;
         put(m_out_, idx.data(), idx.size());
         dalloc(m_flags_, 2 * (size_t)L_.nc);
+        // rows of their own: a stage that starts from U finds it there also after a
+        // read (allocated here, under the library's lock, which a read does not take)
+        dalloc(m_stage_, sizeof(double4) * (size_t)L_.nc);
     }
 
     void reset_state() override { upload_state(); }
@@ -655,16 +658,6 @@ class SolverImpl final : public DeviceSolver {
         check_hip(hipGraphInstantiate(&graph_exec_, graph_, nullptr, nullptr, 0), "hipGraphInstantiate");
     }
 
-    // nc rows for the results on their way out: U, which the next step does not
-    // read while the state is in Uold, else a buffer of its own
-    double4* staging() {
-        if (state_in_uold_) return P_.U;
-        if (!m_stage_.p) {
-            std::lock_guard<std::mutex> lk(runtime_mutex());
-            dalloc(m_stage_, sizeof(double4) * L_.nc);
-        }
-        return m_stage_.as<double4>();
-    }
     // Writes to every page of a result array before the copy that fills it, while
     // the device is still stepping: the copy then meets no page fault.
     static void touch(void* p, size_t bytes) {
