@@ -174,6 +174,12 @@ void launch_gather_state(const double4* src, const int32_t* idx, double4* dst, i
 template <typename R>
 void launch_gather_fields(const DevPtrs<R>& p, const int32_t* idx, double4* W, int8_t* flags, int pairs, int n,
                           hipStream_t s);
+// FP64 at the face centre: stores the face states and limiters that the last
+// reconstruction left out (DevPtrs::fflat).  U: the conserved state that it
+// started from, or null if that is W; dt_ptr: the device time steps of the step
+// that followed (0: none was taken), or null.
+void launch_store_flat(const DevPtrs<double>& p, const double4* U, const double* dt_ptr, double Rg, double gamma,
+                       hipStream_t s);
 // Raises each reconstruction kernel's dynamic-LDS limit to lds minus its static LDS.
 template <typename R> hipError_t set_lds_limits(size_t lds);
 void launch_math_selftest(const double* x, double* out, int n, hipStream_t s);

@@ -1587,6 +1587,11 @@ __device__ __forceinline__ double4 boundary_value(int label, double4 w, double4 
     }
 }
 
+__device__ __forceinline__ double4 primitive_state(const double4& u, double Rgas, double gamma) {
+    const double pr = (gamma - 1.0) * (u.w - 0.5 * (u.y * u.y + u.z * u.z) / u.x);
+    return double4{pr, u.y / u.x, u.z / u.x, pr / (Rgas * u.x)};
+}
+
 // Threads per block of the update, and of the flux pass without the CFL bound
 // (whose tiles of 256 faces carry its partials): 64 where blocks of 256 would
 // leave compute units without one, so that the waves' loads are issued from
@@ -1651,8 +1656,7 @@ __global__ __launch_bounds__(B) void k_update(DevPtrs<R> p, double Rgas, double 
         p.Uold[c] = un;
     else
         p.U[c] = un;
-    const double pr = (gamma - 1.0) * (rhoE - 0.5 * (rhoUx * rhoUx + rhoUy * rhoUy) / rho);
-    const double4 w = double4{pr, rhoUx / rho, rhoUy / rho, pr / (Rgas * rho)};
+    const double4 w = primitive_state(un, Rgas, gamma);
     typename VT<R>::v4 wr;
     wr.x = (R)w.x;
     wr.y = (R)w.y;
@@ -1706,7 +1710,39 @@ __global__ __launch_bounds__(256) void k_gather_fields(DevPtrs<R> p, const int32
     }
 }
 
+// The face states and limiters that the last FP64 face-centre reconstruction
+// left out, for a caller that fetches them.  It started from U where a full step
+// followed it (the second stage's result: the third writes Uold), and from W
+// where none did, or where the step's device time step was 0.
+__global__ __launch_bounds__(256) void k_store_flat(DevPtrs<double> p, const double4* U, const double* dt_ptr,
+                                                    double Rgas, double gamma) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= p.nc || !p.flat_prev[c]) return;
+    const int C = p.ccnt[c], maxC = p.maxC, nf = p.nf;
+    if (p.boundaryFirstOrder)  // cells with a boundary face were stored
+        for (int fi = 0; fi < C; ++fi)
+            if (abs(p.slot_face[sell(c, fi, maxC)]) - 1 >= nf) return;
+    const bool stepped = U && !(dt_ptr && dt_ptr[p.cinst ? p.cinst[c] : 0] == 0.0);
+    const double4 w = stepped ? primitive_state(U[c], Rgas, gamma) : p.W[c];
+    const double2 gp = p.gp[c], gu = p.gu[c], gv = p.gv[c], gT = p.gT[c];
+    p.lim[c] = double4{1.0, 1.0, 1.0, 1.0};
+    for (int fi = 0; fi < C; ++fi) {
+        const int sf = p.slot_face[sell(c, fi, maxC)];
+        const int f = (sf < 0 ? -sf : sf) - 1;
+        if (f >= nf) continue;
+        const double2 d = p.slot_d[sell(c, fi, maxC)];
+        store_face_state(p, 2 * f + (sf < 0),
+                         double4{w.x + gp.x * d.x + gp.y * d.y, w.y + gu.x * d.x + gu.y * d.y,
+                                 w.z + gv.x * d.x + gv.y * d.y, w.w + gT.x * d.x + gT.y * d.y});
+    }
+}
+
 // ---------------------------------------------------------------- launchers
+
+void launch_store_flat(const DevPtrs<double>& p, const double4* U, const double* dt_ptr, double Rg, double gamma,
+                       hipStream_t s) {
+    hipLaunchKernelGGL(k_store_flat, dim3((p.nc + 255) / 256), dim3(256), 0, s, p, U, dt_ptr, Rg, gamma);
+}
 
 void launch_gather_state(const double4* src, const int32_t* idx, double4* dst, int n, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_gather_state, dim3((n + 255) / 256), dim3(256), 0, s, src, idx, dst, n);

@@ -229,6 +229,7 @@ class SolverImpl final : public DeviceSolver {
         // The kernel's last block stores the value in pinned host memory, which
         // the host polls: no copy, and no wait for the launch to retire.  The
         // stored minimum is never NaN.
+        if (flat_from_ == FlatFrom::kDeviceStep) store_flat();  // which reads the step's time step
         volatile double* dt = host_dt_.p;
         *dt = std::nan("");
         launch_cfl<R>(P_, cfg_.R, cfg_.Cv, cfg_.CFL, host_dt_.dev, stream_);
@@ -241,7 +242,7 @@ class SolverImpl final : public DeviceSolver {
     void evolve(double dt) override {
         if (ninst() > 1) throw Error(1, "a batch steps with the device time step only");
         enqueue_stages(dt, nullptr);
-        state_in_uold_ = true;
+        stepped(FlatFrom::kHostStep);
         check_hip(hipGetLastError(), "evolve");
     }
 
@@ -356,6 +357,7 @@ class SolverImpl final : public DeviceSolver {
         launch_bvd<R>(P_, L_.tile, lds_bvd_, stream_);
         launch_flux<R>(P_, cfg_.R, cfg_.Cv, stream_);
         launch_residual_norm<R>(P_, P_.res_part + residual_blocks(L_.nc), stream_);
+        flat_from_ = FlatFrom::kW;
         check_hip(hipGetLastError(), "residual");
         double s = 0.0;
         check_hip(hipMemcpyAsync(&s, P_.res_part + residual_blocks(L_.nc), sizeof(double), hipMemcpyDeviceToHost,
@@ -389,7 +391,7 @@ class SolverImpl final : public DeviceSolver {
             for (int i = 0; i < nsteps; ++i) launch_graph();
         } else {
             for (int i = 0; i < nsteps; ++i) enqueue_stages(0.0, P_.dt);
-            if (nsteps > 0) state_in_uold_ = true;
+            if (nsteps > 0) stepped(FlatFrom::kDeviceStep);
         }
         check_hip(hipEventRecord(ev1_, stream_), "hipEventRecord");
         check_hip(hipEventSynchronize(ev1_), "hipEventSynchronize");
@@ -457,7 +459,7 @@ class SolverImpl final : public DeviceSolver {
         for (int i = 0; i < nsteps; ++i) {
             if (i >= 2) collect(cp[i & 1]);  // step i-2 used this copy
             check_hip(hipGraphLaunch(cp[i & 1].ge, stream_), "hipGraphLaunch");
-            state_in_uold_ = true;
+            stepped(FlatFrom::kDeviceStep);
         }
         check_hip(hipEventRecord(ev1_, stream_), "hipEventRecord");
         for (int i = std::max(0, nsteps - 2); i < nsteps; ++i) collect(cp[i & 1]);
@@ -472,6 +474,7 @@ class SolverImpl final : public DeviceSolver {
     // launches keep transforming the state, so call this after timed work).
     void profile(double* ms, int* count, int reps) override {
         synchronize();
+        run_reconstruct_all();  // on the state that the timed launches below start from
         for (int k = 0; k < kKernKinds; ++k) {
             check_hip(hipEventRecord(ev0_, stream_), "hipEventRecord");
             for (int r = 0; r < reps; ++r) {
@@ -497,14 +500,13 @@ class SolverImpl final : public DeviceSolver {
         count[kKernRecon] = count[kKernBvd] = count[kKernUpdate] = 3;
         count[kKernFlux] = 2;
         count[kKernFluxDt] = count[kKernDtReduce] = 1;
-        for (int k = 0; k < kKernKinds; ++k) {
-        }
     }
 
     const DevLayout& layout() const override { return L_; }
 
     void set_constants(double Rgas, double Cv, double CFL) override {
         if (Rgas == cfg_.R && Cv == cfg_.Cv && CFL == cfg_.CFL) return;
+        store_flat();  // with the constants of the last step
         cfg_.R = Rgas;
         cfg_.Cv = Cv;
         cfg_.CFL = CFL;
@@ -541,6 +543,7 @@ class SolverImpl final : public DeviceSolver {
         pick("lsq", P_.lsq, sizeof(v2) * (size_t)L_.nwaves * L_.maxC * 64);
         if (!src) throw Error(1, std::string("unknown device array ") + what);
         if (bytes != have) throw Error(1, std::string("size mismatch fetching ") + what);
+        if (strcmp(what, "fv") == 0 || strcmp(what, "lim") == 0) store_flat();
         synchronize();
         if (strcmp(what, "fv") == 0 && !P_.fv) {  // (p, Ux, Uy, T) records from the per-variable arrays
             std::vector<R> a[4];
@@ -575,9 +578,7 @@ class SolverImpl final : public DeviceSolver {
     }
 
     void run_stage_kernels(int upto, double dt, int stage) override {
-        DevPtrs<R> P = P_;
-        P.storeFlat = 1;  // every limiter and face state can be fetched afterwards
-        launch_reconstruct<R>(P, L_.tile, lds_recon_, stream_, lanes_);
+        run_reconstruct_all();
         if (upto > 0) launch_bvd<R>(P_, L_.tile, lds_bvd_, stream_);
         if (upto > 1) launch_flux<R>(P_, cfg_.R, cfg_.Cv, stream_);
         if (upto > 2) {
@@ -588,6 +589,31 @@ class SolverImpl final : public DeviceSolver {
     }
 
    private:
+    // FP64 at the face centre: what the last reconstruction started from, where
+    // it left out the limiters and face states of flat cells (kStored: nowhere).
+    // A step's last stage starts from the second stage's result, which is still in U.
+    enum class FlatFrom { kStored, kW, kHostStep, kDeviceStep };
+
+    // A reconstruction that stores every cell's limiters and face states.
+    void run_reconstruct_all() {
+        DevPtrs<R> P = P_;
+        P.storeFlat = 1;
+        launch_reconstruct<R>(P, L_.tile, lds_recon_, stream_, lanes_);
+        flat_from_ = FlatFrom::kStored;
+    }
+    // Completes lim and the face states with the flat cells that the last
+    // reconstruction left out; called before a fetch of them, and before what it
+    // starts from changes other than by a step.
+    void store_flat() {
+        if constexpr (sizeof(R) == 8) {
+            if (flat_from_ == FlatFrom::kStored || L_.ngp) return;
+            const bool step = flat_from_ != FlatFrom::kW;
+            launch_store_flat(P_, step ? P_.U : nullptr, flat_from_ == FlatFrom::kDeviceStep ? P_.dt : nullptr, cfg_.R,
+                              gamma(), stream_);
+            check_hip(hipGetLastError(), "store_flat");
+            flat_from_ = FlatFrom::kStored;
+        }
+    }
     double gamma() const { return cfg_.R / cfg_.Cv + 1.0; }
     // SSP-RK3 Shu-Osher coefficients: the reference's truncated literals
     // (GPUevolve.cu:223-225) or the exact fractions.
@@ -633,6 +659,11 @@ class SolverImpl final : public DeviceSolver {
             mark();
         }
     }
+    // after a full step: where its result is, and what its last reconstruction started from
+    void stepped(FlatFrom from) {
+        state_in_uold_ = true;
+        flat_from_ = from;
+    }
 
     // One graph launch.  At most 2 * kGraphBlock launches are left queued: after
     // every kGraphBlock launches an event is recorded, and before a third
@@ -641,7 +672,7 @@ class SolverImpl final : public DeviceSolver {
     static constexpr int kGraphBlock = 256;
     void launch_graph() {
         check_hip(hipGraphLaunch(graph_exec_, stream_), "hipGraphLaunch");
-        state_in_uold_ = true;
+        stepped(FlatFrom::kDeviceStep);
         if (++launches_ % kGraphBlock) return;
         hipEvent_t& e = evq_[blocks_ & 1];
         if (blocks_ >= 2) check_hip(hipEventSynchronize(e), "hipEventSynchronize");
@@ -687,6 +718,7 @@ class SolverImpl final : public DeviceSolver {
     }
 
     void upload_state() {
+        store_flat();
         state_in_uold_ = false;  // U and Uold both receive the state
         const int nc = L_.nc, nb = L_.nb;
         std::vector<v4> w(nc + nb);
@@ -914,6 +946,7 @@ class SolverImpl final : public DeviceSolver {
     // Uold only (the next step starts from there); a first or second stage
     // writes U.  Host reads take it from state_U().
     bool state_in_uold_ = false;
+    FlatFrom flat_from_ = FlatFrom::kStored;
     double4* state_U() const { return state_in_uold_ ? P_.Uold : P_.U; }
     size_t lds_recon_ = 0, lds_bvd_ = 0, lds_m_off_ = 0, lds_bvd_sten_off_ = 0;
     int lanes_ = 1;  // threads per cell of the reconstruction kernel

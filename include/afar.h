@@ -263,9 +263,7 @@ int afar_solver_sizes(afar_solver* h, int64_t* out);
  * RK stage `stage` with step dt) and copy named device arrays (mesh order):
  * W, U, gp, gu, gv, gT, lim (the raw K5 limiter: the flux pass applies K6's
  * transform as it reads it; -1 marks a first-order cell), smooth, ftype, fv,
- * fvg, flux (FP64 for every face in both precisions), lsq.  In FP64 at the
- * face centre, fv and lim of a cell of uniform temperature (whose face states
- * the flux pass forms itself) are those of the last run_stage call. */
+ * fvg, flux (FP64 for every face in both precisions), lsq. */
 int afar_solver_run_stage(afar_solver* h, int32_t upto, double dt, int32_t stage);
 int afar_solver_fetch(afar_solver* h, const char* name, void* out, size_t bytes);
 void afar_solver_destroy(afar_solver* h);
