@@ -539,11 +539,13 @@ __device__ __forceinline__ int wave_max32(int x, bool m) {
 #ifndef AFAR_RECONQ_WPE_F
 #define AFAR_RECONQ_WPE_F 7
 #endif
-// The instantiations for flux quadrature and (float) for stencils of 20 hold
-// more values and ask for fewer waves, so that they do not spill.
+// The instantiations for flux points and (float) for stencils of 20 hold more
+// values and ask for fewer waves, so that none spills.  With flux points, float
+// stencils past 8 at 5 waves spilled 4 to 8 values: 240k triangles and quads
+// 61.0 us, at 4 waves 54.7.
 template <typename R, bool GP, int MS> struct ReconQWaves {
     static constexpr int value = sizeof(R) == 8 ? AFAR_RECONQ_WPE_D - (GP ? 1 : 0)
-                                                : AFAR_RECONQ_WPE_F - (GP ? 2 : MS > 16 ? 1 : 0);
+                                                : AFAR_RECONQ_WPE_F - (GP ? (MS > 8 ? 3 : 2) : MS > 16 ? 1 : 0);
 };
 #define AFAR_RECONQ_ATTR __attribute__((amdgpu_waves_per_eu(ReconQWaves<R, GP, MS>::value, 8)))
 
@@ -559,6 +561,12 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     // data per slot; the weights are shared within the group by DPP.
     constexpr bool GEO = sizeof(R) == 8 && !GP;
     constexpr bool FLAT = FormsFlat<R, GP>::value;
+    // Flux points: a point's coefficients are requested at once, before its sum,
+    // where the registers for them are there.  A block of 1024 threads leaves a
+    // thread 128, which FP64 stencils past 8 need for the rest: requested at once
+    // they spill 25 values and more, 240k triangles and quads in tiles of 256
+    // 83.8 us, group by group 72.6.
+    constexpr bool AHEAD = !(sizeof(R) == 8 && TILE == 256 && MS > 8);
     extern __shared__ __align__(16) unsigned char smem_raw[];
     v4* sW = reinterpret_cast<v4*>(smem_raw);
     uint16_t* sRows = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
@@ -812,13 +820,14 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     // stencil: the states of a group are requested together, and a cell that
     // has no further members adds -0.0 * 1.
     const int rows = wave_max32(S, live);
-    auto rbf_sum = [&](R own, const G(&g)[NG], v4& o) {
+    auto rbf_sum = [&](R own, auto group, v4& o) {
         o = v4{own * wc.x, own * wc.y, own * wc.z, own * wc.w};
         uint4 ids = row0;
 #pragma unroll
         for (int j = 0; j < NG * V; j += V) {
             if (j < rows) {
                 if (j == 8 || j == 16) ids = row[j / 8];
+                const G g = group(j / V);
                 const unsigned w[4] = {ids.x, ids.y, ids.z, ids.w};
                 v4 m[V];
 #pragma unroll
@@ -828,7 +837,7 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
                 }
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const R coef = CoefGroup<R>::get(g[j / V], i);
+                    const R coef = CoefGroup<R>::get(g, i);
                     o.x += coef * m[i].x;
                     o.y += coef * m[i].y;
                     o.z += coef * m[i].z;
@@ -838,7 +847,7 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
         }
     };
     v4 of;
-    rbf_sum(cf0, cf, of);
+    rbf_sum(cf0, [&](int i) { return cf[i]; }, of);
     const R pf = of.x, uxf = of.y, uyf = of.z, Tf = of.w;
     gradient();
     const R gpx = quad_bcast<0>(gxk), gpy = quad_bcast<0>(gyk), guxx = quad_bcast<1>(gxk),
@@ -872,12 +881,17 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
         if constexpr (GP)
         for (int g = 0; g < p.ngp; ++g) {
             const R* ag = p.rbf_gp + (slice * p.ngp + g) * maxC * p.rbfRow;
+            auto group = [&](int i) { return (reinterpret_cast<const G*>(ag) + i * 64)[a1]; };
             cf0 = ag[a0];
-#pragma unroll
-            for (int i = 0; i < NG; ++i)
-                if (i * V < rows) cf[i] = (reinterpret_cast<const G*>(ag) + i * 64)[a1];
             v4 q;
-            rbf_sum(cf0, cf, q);
+            if constexpr (AHEAD) {
+#pragma unroll
+                for (int i = 0; i < NG; ++i)
+                    if (i * V < rows) cf[i] = group(i);
+                rbf_sum(cf0, [&](int i) { return cf[i]; }, q);
+            } else {
+                rbf_sum(cf0, group, q);
+            }
             const R pg = q.x, uxg = q.y, uyg = q.z, Tg = q.w;
             const v4 dg = p.fgd[(size_t)g * nf + f];
             const R gx = (R)(isNei ? dg.z : dg.x), gy = (R)(isNei ? dg.w : dg.y);
