@@ -222,13 +222,23 @@ __device__ __forceinline__ void store_face_state(const DevPtrs<R>& p, int i, con
     p.fvT[i] = o.w;
 }
 
-// Coefficient i of cell c in row k of K rows per slice (DevLayout::rbf_at).
-template <typename R>
-__device__ __forceinline__ R rbf_at(const R* rbf, int rbfRow, int c, int k, int K, int i) {
-    constexpr int V = 16 / sizeof(R);
-    const R* row = rbf + ((size_t)(c >> 6) * K + k) * rbfRow;
-    return i == 0 ? row[c & 63] : row[64 + ((i - 1) / V * 64 + (c & 63)) * V + (i - 1) % V];
-}
+// A 16-byte group of coefficients.  Rows of single members (4 or 8 bytes a lane
+// and load, up to 17 loads) kept the reconstruction waiting on the loads
+// themselves: 740k mixed 79.3 -> 74.6 us with groups, 1.5M FP64 189 -> 184.5,
+// 20k quads 8.4 -> 7.7, 17k 8.3 -> 7.5.
+template <typename R> struct CoefGroup;
+template <> struct CoefGroup<double> {
+    using type = double2;
+    static __device__ __forceinline__ type splat(double x) { return type{x, x}; }
+    static __device__ __forceinline__ double get(const type& g, int i) { return i ? g.y : g.x; }
+};
+template <> struct CoefGroup<float> {
+    using type = float4;
+    static __device__ __forceinline__ type splat(float x) { return type{x, x, x, x}; }
+    static __device__ __forceinline__ float get(const type& g, int i) {
+        return i == 0 ? g.x : i == 1 ? g.y : i == 2 ? g.z : g.w;
+    }
+};
 
 template <typename R>
 __device__ __forceinline__ void limiter_process(R& lim, R& phif, R phic, R phiMax, R phiMin, R gx, R gy, R dx, R dy) {
@@ -276,6 +286,7 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
     const int tid = threadIdx.x, c = tile * TILE + tid;
     uint16_t* sRows = reinterpret_cast<uint16_t*>(smem_raw + p.lds_sten_off);
     if (c < p.nc) sW[tid] = p.W[c];
+    if (tid == 0) sW[TILE + p.hcap] = v4{(R)1, (R)1, (R)1, (R)1};  // the dummy member
     stage_halo<TILE>(p, tile, tid, TILE, [&](int j, int id) { sW[j] = p.W[id]; });
     {
         const uint4* src = reinterpret_cast<const uint4*>(p.sten + (size_t)tile * TILE * p.stenW);
@@ -379,6 +390,47 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
         return;
     }
 
+    // RBF sum over row k of K per slice (DevLayout::rbf_at): eight members at a
+    // time, their ids one 16-byte word, their coefficients 16-byte groups requested
+    // together; the last group's members past the stencil add -0.0 * 1.  Bound by
+    // its loads: one id and one coefficient a load, which read half or a quarter of
+    // each group, took 123.4 us on 735k triangles and quads in FP32-mixed (so
+    // 106.5; FP64 64.9, 60.0), 23.0 on 180k periodic triangles (21.5; FP64 35.0,
+    // 34.1), at two flux points on 135k 67.1 (48; FP64 73.8, 55.7).
+    constexpr int V = 16 / sizeof(R);
+    using G = typename CoefGroup<R>::type;
+    const uint4* row = reinterpret_cast<const uint4*>(sSt);
+    auto rbf_sum = [&](const R* rbf, int k, int K) {
+        const R* a = rbf + ((size_t)(c >> 6) * K + k) * p.rbfRow;
+        const G* groups = reinterpret_cast<const G*>(a + 64) + (c & 63);
+        const R own = a[c & 63];
+        v4 o = {own * wc.x, own * wc.y, own * wc.z, own * wc.w};
+        for (int j0 = 0; j0 < S; j0 += 8) {
+            const uint4 ids = row[j0 >> 3];
+            const unsigned w[4] = {ids.x, ids.y, ids.z, ids.w};
+            G gs[8 / V];
+#pragma unroll
+            for (int j = 0; j < 8; j += V)
+                if (j0 + j < S) gs[j / V] = groups[(j0 + j) / V * 64];
+#pragma unroll
+            for (int j = 0; j < 8; j += V) {
+                if (j0 + j >= S) break;
+                const G g = gs[j / V];
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const int h = j + i;
+                    const v4 m = sW[(h & 1) ? w[h >> 1] >> 16 : w[h >> 1] & 0xffffu];
+                    const R coef = CoefGroup<R>::get(g, i);
+                    o.x += coef * m.x;
+                    o.y += coef * m.y;
+                    o.z += coef * m.z;
+                    o.w += coef * m.w;
+                }
+            }
+        }
+        return o;
+    };
+
     R limP = 2, limUx = 2, limUy = 2, limT = 2;
     R smoothness = 0;
     int isNotTrouble = 1;
@@ -394,17 +446,8 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
         const R fraction = sqrt(dx * dx + dy * dy) / deltaR;
         const int nbl = sSt[fi];
 
-        auto at = [&](int m) { return rbf_at(p.rbf, p.rbfRow, c, fi, maxC, m); };
-        R coef = at(0);
-        R pf = coef * wc.x, uxf = coef * wc.y, uyf = coef * wc.z, Tf = coef * wc.w;
-        for (int ci = 0; ci < S; ++ci) {
-            const v4 wj = sW[sSt[ci]];
-            coef = at(ci + 1);
-            pf += coef * wj.x;
-            uxf += coef * wj.y;
-            uyf += coef * wj.z;
-            Tf += coef * wj.w;
-        }
+        const v4 of = rbf_sum(p.rbf, fi, maxC);
+        const R pf = of.x, uxf = of.y, uyf = of.z, Tf = of.w;
         v4 o;
         R phif;
         limiter_process(limP, phif, wc.x, pMax, pMin, gpx, gpy, dx, dy);
@@ -422,17 +465,8 @@ __global__ __launch_bounds__(TILE) void k_reconstruct(DevPtrs<R> p) {
         store_face_state(p, 2 * f + isNei, o);
         if constexpr (GP)
         for (int g = 0; g < p.ngp; ++g) {  // flux points (extension), as in k_reconstruct_q
-            auto atg = [&](int m) { return rbf_at(p.rbf_gp, p.rbfRow, c, g * maxC + fi, p.ngp * maxC, m); };
-            R cg = atg(0);
-            R pg = cg * wc.x, uxg = cg * wc.y, uyg = cg * wc.z, Tg = cg * wc.w;
-            for (int ci = 0; ci < S; ++ci) {
-                const v4 wj = sW[sSt[ci]];
-                cg = atg(ci + 1);
-                pg += cg * wj.x;
-                uxg += cg * wj.y;
-                uyg += cg * wj.z;
-                Tg += cg * wj.w;
-            }
+            const v4 q = rbf_sum(p.rbf_gp, g * maxC + fi, p.ngp * maxC);
+            const R pg = q.x, uxg = q.y, uyg = q.z, Tg = q.w;
             const v4 dg = p.fgd[(size_t)g * nf + f];
             const R gx = (R)(isNei ? dg.z : dg.x), gy = (R)(isNei ? dg.w : dg.y);
             v4 og;
@@ -481,24 +515,6 @@ template <int J, typename T> __device__ __forceinline__ T quad_bcast(T x) { retu
 template <int X, typename T> __device__ __forceinline__ T quad_xor(T x) {
     return dpp_move<X == 1 ? 0xB1 : 0x4E>(x);  // quad_perm [1,0,3,2] and [2,3,0,1]
 }
-
-// A 16-byte group of coefficients.  Rows of single members (4 or 8 bytes a lane
-// and load, up to 17 loads) kept the reconstruction waiting on the loads
-// themselves: 740k mixed 79.3 -> 74.6 us with groups, 1.5M FP64 189 -> 184.5,
-// 20k quads 8.4 -> 7.7, 17k 8.3 -> 7.5.
-template <typename R> struct CoefGroup;
-template <> struct CoefGroup<double> {
-    using type = double2;
-    static __device__ __forceinline__ type splat(double x) { return type{x, x}; }
-    static __device__ __forceinline__ double get(const type& g, int i) { return i ? g.y : g.x; }
-};
-template <> struct CoefGroup<float> {
-    using type = float4;
-    static __device__ __forceinline__ type splat(float x) { return type{x, x, x, x}; }
-    static __device__ __forceinline__ float get(const type& g, int i) {
-        return i == 0 ? g.x : i == 1 ? g.y : i == 2 ? g.z : g.w;
-    }
-};
 
 // The largest of the values below 32 that x has in the lanes where m holds (0
 // if there is none): the same in every lane.
