@@ -1979,9 +1979,11 @@ __global__ void k_math_selftest(const double* x, double* out, int n) {
     if (i >= n) return;
     const double v = x[i], w = x[n - 1 - i];
     double c[2], e[2];
-    erfc_exp({w, v}, {w, v}, c, e);  // as the flux calls them: two at once
-    out[4 * i] = e[1];
-    out[4 * i + 1] = c[1];
+    // as the flux calls them: two at once, x[i] the second (even i) or the first
+    const bool first = i & 1;
+    erfc_exp({first ? v : w, first ? w : v}, {first ? v : w, first ? w : v}, c, e);
+    out[4 * i] = first ? e[0] : e[1];
+    out[4 * i + 1] = first ? c[0] : c[1];
     out[4 * i + 2] = sqrt(v < 0 ? -v : v);
     out[4 * i + 3] = 1.0 / v;
 }
@@ -1991,9 +1993,10 @@ __global__ void k_math_selftest_f32(const float* x, float* out, int n) {
     if (i >= n) return;
     const float v = x[i], w = x[n - 1 - i];
     float c[2], e[2];
-    erfc_exp({w, v}, {w, v}, c, e);
-    out[4 * i] = e[1];
-    out[4 * i + 1] = c[1];
+    const bool first = i & 1;
+    erfc_exp({first ? v : w, first ? w : v}, {first ? v : w, first ? w : v}, c, e);
+    out[4 * i] = first ? e[0] : e[1];
+    out[4 * i + 1] = first ? c[0] : c[1];
     out[4 * i + 2] = sqrtf(v < 0 ? -v : v);
     out[4 * i + 3] = 1.0f / v;
 }
