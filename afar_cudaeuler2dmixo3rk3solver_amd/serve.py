@@ -99,15 +99,21 @@ def footprint_bytes(mesh, precision):
     s = mesh.sizes()
     nc, nf, nb, maxS, maxC = s["nc"], s["nf"], s["nb"], s["maxS"], s["maxC"]
     w = 8 if precision == "fp64" else 4
-    nslot = (nc + 63) // 64 * 64 * maxC
-    cell = nc * (4 * w * 4 + 32 * 3 + 8 + 4 * 2 * w + 2 + 2) + (nc + nb) * (4 * w + 1)
-    slots = nslot * (2 * 1 + 4 + 16 + 16 + 2 * w + w) + ((nc + 63) // 64 * 64) * ((maxS + 7) // 8 * 8) * 2
-    rbf = nslot * (maxS + 1) * w
-    faces = nf * (8 + 16 + 2 * 4 * w + 2 + (32 if w == 4 else 0)) + (nf + nb) * 32 + nb * (4 + 1 + 64)
-    # cell and face centres (the FP64 reconstruction, the face passes), the
-    # periodic shifts (counted always: an upper bound), Sf and magSf
-    centres = 16 * (nc + nb + nf + nb) + 16 * nf + 24 * nf
-    return int(cell + slots + rbf + faces + centres + 2 * nc * 4 + (1 << 20))
+    rows = (nc + 63) // 64 * 64
+    nslot = rows * maxC
+    # state, limiters and gradients; flags, stencil sizes and output order
+    cell = (nc + nb) * (4 * w + 1 + 16) + nc * (3 * 32 + 8 + 12 * w + 5 + 6)
+    # stencil ids in whole 16-byte words, per slot its face, geometry, weights and temperature
+    slots = rows * 2 * max(8, (maxS + 7) // 8 * 8) + nslot * (4 + 16 + 6 * w)
+    # RBF coefficients: the cell's own, then the members' in 16-byte groups
+    group = 16 // w
+    rbf = nslot * (1 + (maxS + group - 1) // group * group) * w
+    # cells, area vector and CFL geometry, periodic shift (counted always: an
+    # upper bound), states of both sides, flat-side flags; FP32-mixed: its own
+    # geometry records, temperatures and fluxes
+    faces = nf * (8 + 24 + 16 + 16 + 8 * w + 2 + (32 + 8 + 16 if w == 4 else 0)) + (nf + nb) * (16 + 32) + nb * 69
+    # halo ids (an upper bound: two per cell), partial minima and sums
+    return int(cell + slots + rbf + faces + 2 * nc * 4 + (nf + nb + nc) // 8 + (1 << 20))
 
 
 class Server:
