@@ -86,7 +86,7 @@ struct DevPtrs {
     v2 *gp, *gT, *gu;
 
     v2* gv;
-    uint8_t* flat_prev;        // nc: the cell took the flat branch at the last reconstruction
+    uint8_t* flat_prev;        // nc: the cell took the flat branch at the last reconstruction (what fflat is of)
     // FP64 four-lane reconstruction: the slot geometry and least-squares
     // weights are formed from these instead of read from slot_d, slot_dr, lsq
     const double2* fcen;       // nf+nb face centres
@@ -109,7 +109,7 @@ struct DevPtrs {
     const double2* fcfl;       // nf distance of the cell centres, the owner's share of it
     const float4* fsf32;       // FP32-mixed: nf (Sfx, Sfy, magSf, 0) rounded to float; else null
     const float4* foff32;      // FP32-mixed: nf (dxo, dyo, dxn, dyn) rounded to float; else null
-    double* dt_part;           // dt_cap partial minima of the CFL pass
+    double* dt_part;           // partial minima: kCflBlocks, or two per tile of the flux pass, if more
 
     const R* rbf;              // RBF coefficients: maxC rows per slice (DevLayout::rbf_at)
     const v2* slot_d;          // sliced ELL, face centre - cell centre, in the kernels' precision
@@ -130,7 +130,6 @@ struct DevPtrs {
     v4* fvg;                   // ngp*2*nf reconstructed states at the points, [(g*nf + f)*2 + side]
     double* dt;                // device time step of each instance (ninst)
     unsigned int* dt_count;    // tickets of the CFL pass: kCflGroups + 1 counters 128 bytes apart
-    int dt_cap;                // capacity of dt_part: kCflBlocks or two per flux block, whichever is larger
     // Batches: ninst independent meshes stored one after the other (cells,
     // internal faces, boundary faces each contiguous per instance).  Each has
     // its own CFL time step.  A single mesh is ninst = 1 with cinst = nullptr.
@@ -140,16 +139,15 @@ struct DevPtrs {
     // tctl[4i+2] = steps taken.  The device time step is clipped to land on
     // the end time; once there, steps leave the state unchanged (time step 0).
     double* tctl;
-    double* res_part;          // partial sums of the residual norm (one per update block)
+    double* res_part;          // partial sums of the residual norm (one per 256 cells), then their sum
 };
 
 template <typename R> void launch_lsq(const DevPtrs<R>& p, hipStream_t s);
 // host_dt (optional): pinned host memory that receives the time step too.
 template <typename R>
 void launch_cfl(const DevPtrs<R>& p, double Rg, double Cv, double CFL, double* host_dt, hipStream_t s);
-// lanes: 1 = one thread per cell (any mesh); 4 = four threads per cell;
-// 2 = four threads per cell with the face work compacted (both: meshes whose
-// cells have at most four faces; 2 also tiles of at most 128 cells).
+// lanes: 1 = one thread per cell (any mesh), 4 = four threads per cell (meshes
+// whose cells have at most four faces).
 template <typename R> void launch_reconstruct(const DevPtrs<R>& p, int tile, size_t lds, hipStream_t s, int lanes);
 template <typename R> void launch_bvd(const DevPtrs<R>& p, int tile, size_t lds, hipStream_t s);
 template <typename R> void launch_flux(const DevPtrs<R>& p, double Rg, double Cv, hipStream_t s);
@@ -157,7 +155,7 @@ template <typename R> void launch_flux(const DevPtrs<R>& p, double Rg, double Cv
 // the step starts from) to per-block minima in p.dt_part; launch_dt_reduce
 // then stores their minimum in *p.dt.
 template <typename R> void launch_flux_dt(const DevPtrs<R>& p, double Rg, double Cv, double CFL, hipStream_t s);
-// Tiles of the flux kernels (256 faces each).
+// Tiles of the flux pass that reduces the CFL bound (256 faces each, two partials a tile).
 int flux_tiles(int nf, int nb);
 template <typename R> void launch_dt_reduce(const DevPtrs<R>& p, hipStream_t s);
 // Sum over cells of (density residual / volume)^2 from the current fluxes

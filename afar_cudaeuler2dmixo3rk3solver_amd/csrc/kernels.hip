@@ -167,6 +167,9 @@ __global__ __launch_bounds__(256) void k_cfl(DevPtrs<R> p, double c2T, double CF
         last = 0;
         // The partial is stored past the L2 (agent scope) and is waited for,
         // and read past it below: no fence, which would write the L2 back.
+        // This holds for gfx950, where an agent-scope store that vmcnt has
+        // counted is visible to every XCD; the language's memory model would
+        // ask for release and acquire here.
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (__hip_atomic_fetch_add(mine, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == size - 1) {
             __hip_atomic_store(mine, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -649,8 +652,10 @@ __global__ __launch_bounds__(4 * TILE) AFAR_RECONQ_ATTR void k_reconstruct_q(Dev
     }
     // A cell that took the full path at the previous launch most likely takes
     // it again: its RBF coefficients and centre distance are requested in this
-    // round already (flat_prev only schedules loads; results do not depend on
-    // it).  The row count is the wavefront's: a cell of a shorter stencil reads
+    // round already.  (flat_prev is more than this hint: the writes of fflat
+    // below, which say whose states the face pass forms, are left out where it
+    // says that nothing changed, so both arrays are written by this kernel alone
+    // and together.)  The row count is the wavefront's: a cell of a shorter stencil reads
     // its padding (-0.0), which shares the other cells' 128-byte segments.
     constexpr int V = 16 / sizeof(R), NG = (MS + V - 1) / V;  // members per 16-byte group, groups
     using G = typename CoefGroup<R>::type;
@@ -1801,7 +1806,9 @@ void launch_lsq(const DevPtrs<R>& p, hipStream_t s) {
 // them than 128 break up the streams of the largest meshes (1.5M triangles
 // 1131 us with 128, 1154 with 512; with eighths 1237).  Past 128 a chunk holds
 // at most 12288 cells: 256 FP32-mixed corner flows, 8.2M cells in the largest
-// bucket, 7.54 -> 7.41 ms a step.
+// bucket, 7.54 -> 7.41 ms a step; triangles and quads with 128 chunks and so, FP64:
+// 1.7M cells 978 -> 956 us, 2.3M 1318 -> 1298, 3.8M 2095 -> 2100, 6.6M 3528 -> 3453,
+// FP32-mixed: 965 -> 957, 1325 -> 1316, 2129 -> 2083, 3622 -> 3531.
 template <typename R>
 static DevPtrs<R> mapped(const DevPtrs<R>& p, int n, unsigned& grid, int maxLog = 24) {
     constexpr int kChunkCells = 16384 / sizeof(R), kMaxChunkCells = 12288;
@@ -1875,7 +1882,7 @@ void launch_bvd(const DevPtrs<R>& dev, int tile, size_t lds, hipStream_t s) {
     }
 }
 
-// Whether n threads in blocks of 256 are fewer blocks than the chip has CUs.
+// Whether n threads in blocks of 256 are no more blocks than the chip has CUs (256).
 static bool small_blocks(int n) { return n <= 256 * 256; }
 
 int flux_tiles(int nf, int nb) { return std::max(1, (nf + nb + 255) / 256); }

@@ -906,7 +906,6 @@ class SolverImpl final : public DeviceSolver {
         const size_t dt_bytes = (sizeof(double) * ni + 255) / 256 * 256;
         const size_t count_bytes = ((size_t)(kCflGroups + 1) * 128 + 255) / 256 * 256;
         dalloc(m_dt, dt_bytes + count_bytes + sizeof(double) * dt_cap);
-        P_.dt_cap = dt_cap;
         P_.dt = m_dt.as<double>();
         P_.dt_count = reinterpret_cast<unsigned int*>(m_dt.as<char>() + dt_bytes);
         P_.dt_part = reinterpret_cast<double*>(m_dt.as<char>() + dt_bytes + count_bytes);
