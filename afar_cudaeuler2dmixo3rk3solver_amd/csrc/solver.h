@@ -32,8 +32,8 @@ struct SolverConfig {
 // with every capture makes solvers safe to create, step and destroy from
 // different host threads.  Solver buffers are stream-ordered (hipMallocAsync /
 // hipFreeAsync on the solver's stream) and pinned memory is pooled, never
-// freed, so a destroy waits for its own stream only.  Kernel and graph launches, copies and queries on a solver's own
-// stream do not take the lock.
+// freed, so a destroy waits for its own stream only.  Kernel and graph
+// launches, copies and queries on a solver's own stream do not take the lock.
 std::mutex& runtime_mutex();
 
 // kernel kinds reported by profile()
